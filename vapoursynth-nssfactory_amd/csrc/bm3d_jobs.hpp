@@ -326,6 +326,13 @@ struct WnnmJob {
     FrameRing ring;
     Slots slots;
     long long sum_slot;
+    // Tile path (gram_group_tile_kernel): the tile's numerator partials and
+    // one weight per reference, as FilterJob's; num and den are not used.
+    Grid grid;
+    int range;
+    TileGeom tiles;
+    unsigned long long* part_num;
+    unsigned long long* gweight;
 };
 
 struct WnnmTable {

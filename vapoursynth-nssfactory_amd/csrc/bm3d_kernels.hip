@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "bm3d_jobs.hpp"
 
@@ -3956,6 +3957,411 @@ __global__ __launch_bounds__(64) void ncsr_group_kernel(WnnmTable tab) {
     gram_group_body<N, true>(tab);
 }
 
+// ---------------------------------------------------------------------------
+// Spatial planes of full groups of 8 or 16 blocks of 8 (m = 64, k = N): the
+// arithmetic of gram_group_body, operation for operation (the outputs keep
+// their bits), 64 / N groups to a wave, in registers and on the matrix cores,
+// and the sums of a tile of references in LDS.
+//   unit     16 columns: one group of 16, or two of 8 (column c of group
+//            c >> 3). Four units per wave.
+//   MFMA     v_mfma_f32_16x16x4_f32 sums its four products as a chain of
+//            fused multiply-adds in index order (checked bit for bit against
+//            fmaf chains), so the Gram matrix, the column sums of the
+//            centring, W = V diag(g) V^T (NCSR: V C) and X = A W are MFMAs
+//            with the results of the scalar loops. At N = 8 a product over
+//            columns sums each group's columns (steps s of group s >> 1) in an
+//            accumulator of its own: a neighbour's infinity or NaN stays there.
+//   pixels   lane (kq, n) = 16 kq + n holds pixel 16 t + n of column 4 s + kq:
+//            the B operand of X, and row 4 kq + s of its result is made
+//            column 4 s + kq, so the sums' cells are the gather's. The Gram
+//            operands (column on n, pixel 4 s + kq) go through LDS. X gathers
+//            the pixels again (they are in L1 / L2): holding 64 registers of
+//            them through the rounds would halve the waves per SIMD.
+//   Jacobi   lane i of a group holds row i of G and V, the diagonal apart. A
+//            round's pairs are static, so the column rotations are register
+//            operations with the pair's coefficients broadcast (DPP
+//            row_newbcast, or a swizzle at N = 8); the row rotations read the
+//            partner's row (ds_bpermute). No barriers and no LDS addressing.
+//   sums     the tile's int64 numerators in LDS and one weight per group, as
+//            filter_tile_b8_kernel writes them for finish_tiles_kernel. With
+//            device atomics the kernel is bound by them whatever computes the
+//            groups (77 G/s: 218 us for the 16.6 M of 32 400 groups of 8).
+// Measured on a 1080p plane (MI355X; gram_group_body with its atomics before):
+// groups of 8, step 8 (32 400): 215 -> 59 us, NCSR 225 -> 67 us; groups of 16,
+// step 4 (128 855): 3 732 -> 984 us, there bound by VALU issue in the rounds
+// (96 % of the SIMDs' cycles); the smaller launch holds four waves per SIMD and
+// waits a third of its cycles.
+// ---------------------------------------------------------------------------
+
+// Calls f(integral_constant<0>) .. f(integral_constant<N - 1>).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// rr_partner for a full group.
+template <int N>
+__host__ __device__ constexpr int rr_pair(int i, int r) {
+    if (i == N - 1) return r;
+    if (i == r) return N - 1;
+    return (2 * r - i + N - 1) % (N - 1);
+}
+
+// v of lane P of the caller's group of N lanes.
+template <int N, int P>
+__device__ __forceinline__ float group_lane_f32(float v) {
+    if constexpr (N == 16)
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + P, 0xf, 0xf, true));
+    else
+        return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x18 | (P << 5)));
+}
+
+// Round R of a sweep over the lanes' rows g, v and diagonal d; oi the lane's
+// row, lane4 and partner4 its lane and its partner's, times four. False, and nothing changed,
+// when no pair of the wave rotates.
+template <int N, int R>
+__device__ __forceinline__ bool jacobi_round(float (&g)[N], float (&v)[N], float& d, int oi, int lane4, int partner4,
+                                             float floor_abs) {
+    auto from_partner = [&](float x) {
+        return __int_as_float(__builtin_amdgcn_ds_bpermute(partner4, __float_as_int(x)));
+    };
+    float own = g[rr_pair<N>(0, R)];  // G[i][partner]
+#pragma unroll
+    for (int j = 1; j < N; ++j) own = oi == j ? g[rr_pair<N>(j, R)] : own;
+    const float dp = from_partner(d), other = from_partner(own);
+    // the lane of the smaller index is p (g_pp, g_pq), the other q
+    const bool low = lane4 < partner4;
+    const float apq = low ? own : other, app = low ? d : dp, aqq = low ? dp : d;
+    const float apq2 = apq * apq;
+    const bool rot = fabsf(apq) > floor_abs && apq2 > kWnnmTol * kWnnmTol * fabsf(app * aqq);
+    if (!__any(rot)) return false;
+    const float delta = (aqq - app) * 0.5f;
+    const float root = __builtin_amdgcn_sqrtf(fmaf(delta, delta, apq2));
+    float tn = apq * __builtin_amdgcn_rcpf(delta + copysignf(root, delta));
+    float c = __builtin_amdgcn_rsqf(fmaf(tn, tn, 1.f));
+    float sn = tn * c;
+    c = rot ? c : 1.f;
+    sn = rot ? sn : 0.f;
+    tn = rot ? tn : 0.f;
+    const float sa = low ? -sn : sn, ta = low ? -tn : tn;
+    float t[N];
+    static_for<N>([&](auto pc) {
+        constexpr int p = decltype(pc)::value, q = rr_pair<N>(p, R);
+        if constexpr (p < q) {
+            const float cb = group_lane_f32<N, p>(c), sb = group_lane_f32<N, p>(sa);
+            const float g0 = g[p], g1 = g[q], v0 = v[p], v1 = v[q];
+            t[p] = fmaf(cb, g0, sb * g1);
+            t[q] = fmaf(cb, g1, -(sb * g0));
+            v[p] = fmaf(cb, v0, sb * v1);
+            v[q] = fmaf(cb, v1, -(sb * v0));
+        }
+    });
+    const float pair = sa != 0.f ? 0.f : own;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        const float x = fmaf(c, t[j], sa * from_partner(t[j]));
+        g[j] = oi == rr_pair<N>(j, R) ? pair : x;
+    }
+    d = fmaf(ta, own, d);
+    return true;
+}
+
+// Floats of a wave's scratch: the unit matrices, a unit's half columns (NCSR:
+// the code rows of all units) and two vectors.
+inline constexpr int kGramP = 17;   // pitch of a unit's matrices
+inline constexpr int kGramPx = 44;  // pitch of a half column's 32 pixels: both operand reads spread over the banks
+inline constexpr int kGramMat = 4 * 16 * kGramP;
+inline constexpr int kGramScratch = 2 * kGramMat + 128;
+
+// One workgroup of four waves per tile of at most 4 (64 / N) references. LDS:
+// the waves' scratch, then (over it) the tile's numerator sums.
+template <int N, bool NCSR>
+__global__ __launch_bounds__(256, 4) void gram_group_tile_kernel(WnnmTable tab) {
+    extern __shared__ __align__(16) unsigned long long acc[];
+    constexpr int GW = 64 / N;   // groups of a wave
+    constexpr int HN = 16 / N;   // groups of a unit
+    constexpr int P = kGramP, PX = kGramPx;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 15, kq = lane >> 4;
+    const int lb = xcd_block();
+    const WnnmJob& jb = tab.job[find_job(tab, lb)];
+    const TileGeom& tg = jb.tiles;
+    const int tile = lb - jb.wg_begin, tx = tile % tg.ntx, ty = tile / tg.ntx;
+    const int aw = tg.aw, ah = tg.ah;
+    const int ax0 = tg.ax0(tx, jb.width, 8, jb.grid.step, jb.range);
+    const int ay0 = tg.ay0(ty, jb.height, 8, jb.grid.step, jb.range);
+    const int i_begin = tx * tg.tw, j_begin = ty * tg.th;
+    const int ni = min(tg.tw, jb.grid.nx - i_begin), ngroups = ni * min(tg.th, jb.grid.ny - j_begin);
+    const int g0 = wave * GW;
+    float* mat = reinterpret_cast<float*>(acc) + wave * kGramScratch;  // Gram, then V, then W
+    float* px = mat + kGramMat;
+    float* vec = px + kGramMat;
+    float* vec2 = vec + 64;
+    // Group (of the tile) of column c of unit u; groups past the tile's last
+    // repeat it and add nothing.
+    auto group_of = [&](int u, int c) { return g0 + u * HN + c / N; };
+    auto ref_of = [&](int g) {
+        const int q = min(g, ngroups - 1), gj = q / ni;
+        return (j_begin + gj) * jb.grid.nx + i_begin + (q - gj * ni);
+    };
+    auto record = [&](int u, int c) {
+        return jb.matches[static_cast<size_t>(ref_of(group_of(u, c))) * N + c % N];
+    };
+    // Pixel 16 t + n of columns 4 s + kq of a unit.
+    auto gather = [&](const MatchRec (&rec)[4], float (&b)[4][4]) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const float* p = jb.src + static_cast<size_t>(rec[s].y + (n >> 3)) * jb.stride + rec[s].x + (n & 7);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) b[t][s] = p[static_cast<size_t>(2 * t) * jb.stride];
+        }
+    };
+    // Row centring (src/cpu/common/group_center.cpp:15-58) of one pixel tile:
+    // a row of ones times the columns sums them in order (every row of the
+    // result is alike); the means (0 without centring) are subtracted.
+    auto centre = [&](float (&b)[4], float (&mu)[HN]) {
+#pragma unroll
+        for (int h = 0; h < HN; ++h) mu[h] = 0.f;
+        if (!jb.residual) return;
+        f32x4 sum[HN];
+#pragma unroll
+        for (int h = 0; h < HN; ++h) sum[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            sum[4 * s / N] = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, b[s], sum[4 * s / N], 0, 0, 0);
+#pragma unroll
+        for (int h = 0; h < HN; ++h) mu[h] = sum[h][0] * (1.f / N);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) b[s] -= mu[4 * s / N];
+    };
+
+    float wt = 1.f;    // of the lane's group
+    float wv[4][4];    // W's A operand: rows 4 s + kq, column orow
+    const int orow = 4 * (n & 3) + (n >> 2);
+    if (g0 < ngroups) {
+        {
+            MatchRec rec[4][4];
+            float b[4][4][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) rec[u][s] = record(u, 4 * s + kq);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) gather(rec[u], b[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                f32x4 gram = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        float mu[HN];
+                        centre(b[u][2 * half + t], mu);
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) px[(4 * s + kq) * PX + 16 * t + n] = b[u][2 * half + t][s];
+                    }
+                    wave_sync();
+#pragma unroll
+                    for (int s = 0; s < 8; ++s) {
+                        const float x = px[n * PX + 4 * s + kq];
+                        gram = __builtin_amdgcn_mfma_f32_16x16x4f32(x, x, gram, 0, 0, 0);
+                    }
+                    wave_sync();
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mat[u * 16 * P + (4 * kq + j) * P + n] = gram[j];
+            }
+            wave_sync();
+        }
+
+        // Jacobi: lane = (group, row).
+        const int oi = lane & (N - 1), base = lane & ~(N - 1);
+        float* row = mat + lane / 16 * (16 * P) + (lane & 15) * P + (lane & 15 & ~(N - 1));
+        float d = 0.f;
+        {
+            float g[N], v[N];
+            float trace = 0.f;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                g[j] = row[j];
+                v[j] = oi == j ? 1.f : 0.f;
+                d = oi == j ? g[j] : d;
+            }
+            static_for<N>([&](auto jc) { trace += group_lane_f32<N, decltype(jc)::value>(d); });
+            const float floor_abs = kWnnmFloor * trace;
+            // A group whose trace is not finite never rotates; where a
+            // neighbour in the wave does, its rows are put back below.
+            const bool frozen = !(fabsf(floor_abs) < __builtin_inff());
+            const float d0 = d;
+            uint32_t partners[(N + 2) / 4];
+#pragma unroll
+            for (int r = 0; r < N - 1; ++r) {
+                const uint32_t at = static_cast<uint32_t>(base | rr_partner(oi, r, N)) << (8 * (r & 3));
+                partners[r >> 2] = (r & 3) == 0 ? at : partners[r >> 2] | at;
+            }
+            for (int sweep = 0; sweep < kWnnmSweeps; ++sweep) {
+                bool rotated = false;
+                static_for<N - 1>([&](auto rc) {
+                    constexpr int r = decltype(rc)::value;
+                    const int partner4 = static_cast<int>((partners[r >> 2] >> (8 * (r & 3))) & 63u) << 2;
+                    rotated |= jacobi_round<N, r>(g, v, d, oi, lane << 2, partner4, floor_abs);
+                });
+                if (!rotated) break;
+            }
+            d = frozen ? d0 : d;
+#pragma unroll
+            for (int j = 0; j < N; ++j) row[j] = frozen ? (oi == j ? 1.f : 0.f) : v[j];
+        }
+
+        // Spectrum: s_j, lane = eigenvalue.
+        const float sj = sqrtf(fmaxf(d, 0.f));
+        vec[lane] = sj;
+        // sums over the unit's indices l = 4 s + kq, a group's steps apart;
+        // the rows 4 kq + j of the result from their own group's sums
+        auto product = [&](auto left, auto right) {
+            f32x4 sum[HN];
+#pragma unroll
+            for (int h = 0; h < HN; ++h) sum[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                sum[4 * s / N] =
+                    __builtin_amdgcn_mfma_f32_16x16x4f32(left(4 * s + kq), right(4 * s + kq), sum[4 * s / N], 0, 0, 0);
+            f32x4 out = sum[0];
+            if constexpr (HN == 2)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) out[j] = kq >= 2 ? sum[1][j] : sum[0][j];
+            return out;
+        };
+        if constexpr (NCSR) {
+            // beta is rounded before it is added, as there
+#pragma clang fp contract(off)
+            // The code rows of gram_group_body, C[i][j] over s_i, into px.
+            const float sg = jb.sigma;
+            const float h = fmaxf(2.f * 64.f * sg * sg, 1e-12f);
+            vec2[lane] = expf(-(oi > 0 ? __uint_as_float(record(lane >> 4, lane & 15).dist) : 0.f) / h);
+            wave_sync();
+            float wsum = 0.f;
+#pragma unroll
+            for (int j = 0; j < N; ++j) wsum += vec2[base + j];
+            const bool unit = !(wsum > 0.f);
+            const float inverse = 1.f / (unit ? static_cast<float>(N) : wsum);
+            const float* vcol = mat + lane / 16 * (16 * P) + (lane & 15 & ~(N - 1)) * P + (lane & 15);
+            float code[N], beta = 0.f, moment = 0.f;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                code[j] = vcol[j * P];
+                beta = fmaf(unit ? 1.f : vec2[base + j], sj * code[j], beta);
+            }
+            beta *= inverse;
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const float e = fmaf(sj, code[j], -beta);
+                moment = fmaf(e, e, moment);
+            }
+            const float tau = 2.8284271247461903f * sg * sg / (sqrtf(moment / static_cast<float>(N)) + 1e-12f);
+            const float inv_s = 1.f / sj;
+            float* crow = px + lane / 16 * (16 * P) + (lane & 15) * P + (lane & 15 & ~(N - 1));
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                const float e = fmaf(sj, code[j], -beta), ae = fabsf(e);
+                const float x = ((ae > tau ? copysignf(ae - tau, e) : 0.f) + beta) * inv_s;
+                crow[j] = !(sg > 0.f) ? code[j] : sj > 0.f ? x : 0.f;
+            }
+            wave_sync();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float* vu = mat + u * 16 * P + n * P;
+                const float* cu = px + u * 16 * P + n;
+                const f32x4 m = product([&](int l) { return vu[l]; }, [&](int l) { return cu[l * P]; });
+                wave_sync();
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mat[u * 16 * P + (4 * kq + j) * P + n] = m[j];
+            }
+        } else {
+            // Gains of gram_group_body; only the first place matters there.
+            wave_sync();
+            bool keep = false;
+            float gj = 0.f;
+            if (!jb.residual) {
+                int place = 0;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const float si = vec[base + i];
+                    place += (si > sj || (si == sj && i < oi)) ? 1 : 0;
+                }
+                keep = place == 0;
+                gj = keep ? 1.f : 0.f;
+            }
+            const float constant = 8.f * sqrtf(2.f * static_cast<float>(N)) * jb.sigma * jb.sigma;
+            const float tmp = fmaf(sj, sj, -constant);
+            if (!keep && tmp > 0.f) {
+                gj = ((sj + sqrtf(tmp)) * 0.5f) / sj;
+                keep = true;
+            }
+            const int kept = __popc(static_cast<uint32_t>(__ballot(keep) >> base) & ((1u << N) - 1u));
+            wt = jb.adaptive && kept > 0 ? 1.f / static_cast<float>(kept) : 1.f;
+            vec2[lane] = gj;
+            wave_sync();
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float* vu = mat + u * 16 * P + n * P;
+                const float* gu = vec2 + u * 16;
+                const f32x4 w = product([&](int l) { return vu[l] * gu[l]; }, [&](int l) { return vu[l]; });
+                wave_sync();
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mat[u * 16 * P + (4 * kq + j) * P + n] = w[j];
+            }
+        }
+        wave_sync();
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) wv[u][s] = mat[u * 16 * P + (4 * s + kq) * P + orow];
+        if (oi == 0 && g0 + lane / N < ngroups) jb.gweight[ref_of(g0 + lane / N)] = to_fixed(wt);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < aw * ah; e += 256) acc[e] = 0ull;
+    __syncthreads();
+
+    // X[c][e] = sum_i W[i][c] A[i][e] plus the centre: row 4 kq + j of the
+    // result is column c = 4 j + kq.
+    if (g0 < ngroups) {
+        MatchRec rec[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) rec[u][s] = record(u, 4 * s + kq);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            float b[4][4];
+            gather(rec[u], b);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                f32x4 x[HN];
+                float mu[HN];
+                centre(b[t], mu);
+#pragma unroll
+                for (int h = 0; h < HN; ++h) x[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    x[4 * s / N] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][s], b[t][s], x[4 * s / N], 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int h = 4 * j / N;
+                    const float w = lane_f32(wt, N * (u * HN + h));
+                    unsigned long long* cell = acc + (rec[u][j].y - ay0 + 2 * t + (n >> 3)) * aw + rec[u][j].x - ax0 + (n & 7);
+                    if (g0 + u * HN + h < ngroups) lds_add(cell, to_fixed(w * (x[h][j] + mu[h])));
+                }
+            }
+        }
+    }
+    __syncthreads();
+    partials_out(aw, ah, tg.pitch, acc, jb.part_num + static_cast<size_t>(tile) * tg.pitch * ah + (ax0 & 3));
+}
+
 // NCSR rounds after the first: est += delta (noisy - est)
 // (src/cpu/common/iter_regularize.cpp:15-39). 64 x 4 pixels per block.
 __global__ __launch_bounds__(256) void regularize_kernel(float* est, int est_stride, const float* noisy,
@@ -4471,6 +4877,33 @@ static hipError_t launch_gram_groups(const WnnmTable& t, int total_wg, size_t ld
         wnnm_group_kernel<N><<<total_wg, 64, lds, s>>>(t);
     }
     return hipGetLastError();
+}
+
+// LDS of gram_group_tile_kernel for a plane whose every reference has a full
+// group (the smallest window, a corner's, holds it) in tiles of g; 0 where
+// the kernel does not serve the shape.
+size_t gram_tile_lds_bytes(int block, int group, int range, int width, int height, const TileGeom& g) {
+    if (block != 8 || (group != 8 && group != 16) || g.tw * g.th > 4 * (64 / group)) return 0;
+    const long long w = std::min(range, width - block) + 1, h = std::min(range, height - block) + 1;
+    if (w * h < group) return 0;
+    return std::max(static_cast<size_t>(g.aw) * g.ah * 8, static_cast<size_t>(4 * kGramScratch) * 4);
+}
+
+hipError_t launch_wnnm_tiles(const WnnmTable& t, int total_wg, size_t lds, bool ncsr, hipStream_t s) {
+    if (launch_fault()) return hipErrorLaunchFailure;
+    const int group = t.job[0].group;
+    for (int j = 0; j < t.n; ++j) {
+        const WnnmJob& q = t.job[j];
+        const size_t need = gram_tile_lds_bytes(q.block, q.group, q.range, q.width, q.height, q.tiles);
+        if (q.group != group || need == 0 || need > lds || q.temporal) return hipErrorInvalidValue;
+    }
+    auto launch = [&](auto kernel) {
+        allow_lds(kernel, lds);
+        kernel<<<total_wg, 256, lds, s>>>(t);
+        return hipGetLastError();
+    };
+    if (group == 8) return ncsr ? launch(&gram_group_tile_kernel<8, true>) : launch(&gram_group_tile_kernel<8, false>);
+    return ncsr ? launch(&gram_group_tile_kernel<16, true>) : launch(&gram_group_tile_kernel<16, false>);
 }
 
 hipError_t launch_wnnm(const WnnmTable& t, int total_wg, bool ncsr, hipStream_t s) {

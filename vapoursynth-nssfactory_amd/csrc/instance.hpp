@@ -79,6 +79,11 @@ hipError_t launch_vaggregate(const VAggJob& jb, hipStream_t s);
 size_t wnnm_lds_bytes(int block, int group);
 // ncsr: the NCSR code shrink on the same eigenbasis instead of WNNM's.
 hipError_t launch_wnnm(const WnnmTable& t, int total_wg, bool ncsr, hipStream_t s);
+// The same on tiles of references, for full groups of 8 or 16 blocks of 8 of
+// spatial planes: LDS bytes of a plane's tiles (0 where it does not serve the
+// shape) and the launch.
+size_t gram_tile_lds_bytes(int block, int group, int range, int width, int height, const TileGeom& g);
+hipError_t launch_wnnm_tiles(const WnnmTable& t, int total_wg, size_t lds, bool ncsr, hipStream_t s);
 hipError_t launch_regularize(float* est, int est_stride, const float* noisy, int noisy_stride, int width, int height,
                              float delta, hipStream_t s);
 // The matcher kind for one plane (3 MFMA, 2 run, 1 wave with the window in

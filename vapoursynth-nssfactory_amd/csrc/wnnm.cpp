@@ -5,14 +5,17 @@
 // radius 0): clear the plane's fixed-point sums, match every raster reference
 // on rclip (or src) with the BM3D matchers, shrink each group and add it into
 // the sums (wnnm_group_kernel), then finish dst = num / den, or src where no
-// patch landed (the atomic path's corner finish). A plane with sigma 0 is
-// copied (src/host/filter_wnnm.cpp:236-246).
+// patch landed (the atomic path's corner finish). Full groups of 8 or 16
+// blocks of 8 take the tile path instead (gram_group_tile_kernel and the tile
+// finish; nothing to clear). A plane with sigma 0 is copied
+// (src/host/filter_wnnm.cpp:236-246).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <mutex>
 #include <new>
 #include <string>
+#include <utility>
 
 #include "instance.hpp"
 
@@ -34,12 +37,17 @@ struct nss_hip_wnnm {
         int* counts = nullptr;
         unsigned long long* num = nullptr;  // 2 radius + 1 slices when temporal
         unsigned long long* den = nullptr;
+        TileGeom tiles{};                    // tile path
+        unsigned long long* part = nullptr;  // its numerator partials, then one weight per reference
+        size_t part_elems = 0;
         float* est = nullptr;  // NCSR estimate, width floats per row; a ring like win when temporal
         // Temporal: the window's frames (frame f at (f % (2 radius + 1)) * pixels),
         // and rclip's when one is given.
         float* win = nullptr;
         float* mwin = nullptr;
     } pl[3];
+    bool tiled = false;   // the tile path serves every active plane
+    size_t tile_lds = 0;
     long long bytes = 0;
     std::mutex mu;  // temporal calls: one at a time (the window and sums are shared)
 };
@@ -56,6 +64,8 @@ void release(nss_hip_wnnm* h) {
         if (q.num) dev_free(q.num);
         if (q.den) dev_free(q.den);
         if (q.est) dev_free(q.est);
+        if (q.part) dev_free(q.part);
+        q.part = nullptr;
         dev_free(q.win);
         dev_free(q.mwin);
         q.win = q.mwin = nullptr;
@@ -65,6 +75,33 @@ void release(nss_hip_wnnm* h) {
         q.num = nullptr;
         q.den = nullptr;
     }
+}
+
+// The tile path's plan (radius 0), when it serves every active plane: the
+// largest tile whose sums leave two workgroups per CU, in shapes that fill the
+// kernel's four waves (64 / group groups each). 1080p, groups of 8 at range 7:
+// 8 x 4 references 59 us; 4 x 4, two waves of each workgroup idle, 83 us.
+bool plan_tiles(nss_hip_wnnm* h) {
+    const nss_hip_wnnm_params& p = h->p;
+    const int per_tile = 4 * (64 / std::max(p.group_size, 1));
+    for (const auto& sh : {std::pair<int, int>{8, 4}, {4, 4}, {4, 2}}) {
+        if (p.radius > 0 || sh.first * sh.second > per_tile) continue;
+        size_t lds = 0;
+        bool ok = true;
+        for (int i = 0; i < h->vi.num_planes; ++i) {
+            auto& q = h->pl[i];
+            if (!q.active) continue;
+            q.tiles = make_tiles(q.grid, sh.first, sh.second, p.block_size, p.bm_range);
+            const size_t need =
+                gram_tile_lds_bytes(p.block_size, p.group_size, p.bm_range, q.width, q.height, q.tiles);
+            ok &= need != 0;
+            lds = std::max(lds, need);
+        }
+        if (!ok || lds > kTileLdsBudget) continue;
+        h->tile_lds = lds;
+        return true;
+    }
+    return false;
 }
 
 // Buffers of every active plane; h->ncsr and the parameters are set.
@@ -99,35 +136,63 @@ int init_instance(nss_hip_wnnm* h, const nss_hip_wnnm_params& p, const nss_hip_v
         q.height = info->height >> (i ? info->sub_sampling_h : 0);
         q.active = p.sigma[i] != 0.f;
         if (!q.active) continue;
-        if (q.width < p.block_size || q.height < p.block_size) {
-            release(h);
+        if (q.width < p.block_size || q.height < p.block_size)
             return fail(NSS_HIP_INVALID_INPUT, "nss: selected plane is smaller than block_size");
-        }
         q.grid = make_grid(q.width, q.height, p.block_size, p.block_step);
         q.nref = q.grid.nx * q.grid.ny;
+    }
+    // The instance's device memory on the tile path (the frame-sized sums
+    // replaced by the tiles' partials), or on the atomic path: where a memory
+    // limit holds only the smaller of the two, that one.
+    auto sizes = [&](const nss_hip_wnnm::Plane& q, size_t (&out)[7]) {
         const size_t pixels = static_cast<size_t>(q.width) * q.height;
-        const size_t rec_bytes = static_cast<size_t>(q.nref) * p.group_size * sizeof(MatchRec);
-        const size_t cnt_bytes = static_cast<size_t>(q.nref) * sizeof(int);
         const size_t slices = 2 * static_cast<size_t>(p.radius) + 1;
-        const size_t sum_bytes = slices * pixels * sizeof(unsigned long long);
-        const size_t est_bytes = h->ncsr ? slices * pixels * sizeof(float) : 0;
-        const size_t win_bytes = p.radius > 0 ? slices * pixels * sizeof(float) : 0;
-        const size_t mwin_bytes = p.radius > 0 && p.has_rclip ? win_bytes : 0;
-        h->bytes += static_cast<long long>(rec_bytes + cnt_bytes + 2 * sum_bytes + est_bytes + win_bytes + mwin_bytes);
-        if ((e = dev_alloc(&q.recs, rec_bytes)) != hipSuccess || (e = dev_alloc(&q.counts, cnt_bytes)) != hipSuccess ||
-            (e = dev_alloc(&q.num, sum_bytes)) != hipSuccess || (e = dev_alloc(&q.den, sum_bytes)) != hipSuccess ||
-            (h->ncsr && (e = dev_alloc(&q.est, est_bytes)) != hipSuccess) ||
-            (win_bytes && (e = dev_alloc(&q.win, win_bytes)) != hipSuccess) ||
-            (mwin_bytes && (e = dev_alloc(&q.mwin, mwin_bytes)) != hipSuccess)) {
+        out[0] = static_cast<size_t>(q.nref) * p.group_size * sizeof(MatchRec);
+        out[1] = static_cast<size_t>(q.nref) * sizeof(int);
+        out[2] = h->tiled ? 0 : 2 * slices * pixels * sizeof(unsigned long long);
+        out[3] = h->tiled ? (static_cast<size_t>(q.tiles.ntx) * q.tiles.nty * q.tiles.pitch * q.tiles.ah + q.nref) *
+                                sizeof(unsigned long long)
+                          : 0;
+        out[4] = h->ncsr ? slices * pixels * sizeof(float) : 0;
+        out[5] = p.radius > 0 ? slices * pixels * sizeof(float) : 0;
+        out[6] = p.radius > 0 && p.has_rclip ? out[5] : 0;
+    };
+    auto total = [&]() {
+        long long bytes = 0;
+        for (int i = 0; i < info->num_planes; ++i) {
+            if (!h->pl[i].active) continue;
+            size_t z[7];
+            sizes(h->pl[i], z);
+            for (size_t b : z) bytes += static_cast<long long>(b);
+        }
+        return bytes;
+    };
+    const long long limit = p.memory_limit_mb > 0 ? static_cast<long long>(p.memory_limit_mb) << 20 : 0;
+    h->tiled = plan_tiles(h);
+    h->bytes = total();
+    if (h->tiled && limit && h->bytes > limit) {
+        h->tiled = false;
+        h->bytes = total();
+    }
+    if (limit && h->bytes > limit) {
+        const long long need = (h->bytes + (1ll << 20) - 1) >> 20;
+        return fail(NSS_HIP_INVALID_INPUT, ns + ": memory_limit_mb is too small for this clip: the instance needs at "
+                                                "least " + std::to_string(need) + " MiB");
+    }
+    for (int i = 0; i < info->num_planes; ++i) {
+        auto& q = h->pl[i];
+        if (!q.active) continue;
+        size_t z[7];
+        sizes(q, z);
+        q.part_elems = z[3] ? z[3] / sizeof(unsigned long long) - q.nref : 0;
+        if ((e = dev_alloc(&q.recs, z[0])) != hipSuccess || (e = dev_alloc(&q.counts, z[1])) != hipSuccess ||
+            (z[2] && ((e = dev_alloc(&q.num, z[2] / 2)) != hipSuccess || (e = dev_alloc(&q.den, z[2] / 2)) != hipSuccess)) ||
+            (z[3] && (e = dev_alloc(&q.part, z[3])) != hipSuccess) || (z[4] && (e = dev_alloc(&q.est, z[4])) != hipSuccess) ||
+            (z[5] && (e = dev_alloc(&q.win, z[5])) != hipSuccess) ||
+            (z[6] && (e = dev_alloc(&q.mwin, z[6])) != hipSuccess)) {
             release(h);
             return hip_fail(e, "group filter buffers");
         }
-    }
-    if (p.memory_limit_mb > 0 && h->bytes > static_cast<long long>(p.memory_limit_mb) << 20) {
-        const long long need = (h->bytes + (1ll << 20) - 1) >> 20;
-        release(h);
-        return fail(NSS_HIP_INVALID_INPUT, ns + ": memory_limit_mb is too small for this clip: the instance needs at "
-                                                "least " + std::to_string(need) + " MiB");
     }
     return NSS_HIP_OK;
 }
@@ -147,13 +212,14 @@ int group_round(nss_hip_wnnm* h, const float* const* mplane, const int* mstride,
         const auto& q = h->pl[i];
         if (!q.active) continue;
         const long long pixels = static_cast<long long>(q.width) * q.height;
-        for (unsigned long long* buf : {q.num, q.den}) {
-            ZeroJob& z = zt.job[zt.n++];
-            z.p = buf;
-            z.count = pixels;
-            z.wg_begin = zero_wg;
-            zero_wg += static_cast<int>((pixels + 1023) / 1024);
-        }
+        if (!h->tiled)
+            for (unsigned long long* buf : {q.num, q.den}) {
+                ZeroJob& z = zt.job[zt.n++];
+                z.p = buf;
+                z.count = pixels;
+                z.wg_begin = zero_wg;
+                zero_wg += static_cast<int>((pixels + 1023) / 1024);
+            }
         WnnmJob& w = wt.job[wt.n++];
         w.src = gsrc[i];
         w.width = q.width;
@@ -170,7 +236,12 @@ int group_round(nss_hip_wnnm* h, const float* const* mplane, const int* mstride,
         w.counts = q.counts;
         w.num = q.num;
         w.den = q.den;
-        wnnm_wg += q.nref;
+        w.grid = q.grid;
+        w.range = p.bm_range;
+        w.tiles = q.tiles;
+        w.part_num = q.part;
+        w.gweight = q.part ? q.part + q.part_elems : nullptr;
+        wnnm_wg += h->tiled ? q.tiles.ntx * q.tiles.nty : q.nref;
         FinishJob& f = ft.job[ft.n++];
         f.num = q.num;
         f.den = q.den;
@@ -182,12 +253,21 @@ int group_round(nss_hip_wnnm* h, const float* const* mplane, const int* mstride,
         f.height = q.height;
         f.sstride = fsstride[i];
         f.dstride = fdstride[i];
-        f.tiles_x = (q.width + 15) / 16;
+        f.exact_num = reinterpret_cast<const long long*>(q.part);
+        f.matches = q.recs;
+        f.counts = q.counts;
+        f.gweight = w.gweight;
+        f.grid = q.grid;
+        f.group = p.group_size;
+        f.tiles = q.tiles;
+        f.step = p.block_step;
+        f.range = p.bm_range;
+        f.tiles_x = h->tiled ? (q.width + 63) / 64 : (q.width + 15) / 16;
         f.wg_begin = finish_wg;
         finish_wg += f.tiles_x * ((q.height + 15) / 16);
     }
     if (wt.n == 0) return NSS_HIP_OK;
-    if ((e = launch_zero(zt, zero_wg, s)) != hipSuccess) return hip_fail(e, "group filter clear");
+    if (zt.n && (e = launch_zero(zt, zero_wg, s)) != hipSuccess) return hip_fail(e, "group filter clear");
     for (int i = 0; i < h->vi.num_planes; ++i) {
         const auto& q = h->pl[i];
         if (!q.active) continue;
@@ -210,8 +290,9 @@ int group_round(nss_hip_wnnm* h, const float* const* mplane, const int* mstride,
         if ((e = launch_match(p.block_size, mt, match_workgroups(kind, q.grid), lds, kind, s)) != hipSuccess)
             return hip_fail(e, "group filter match launch");
     }
-    if ((e = launch_wnnm(wt, wnnm_wg, h->ncsr, s)) != hipSuccess) return hip_fail(e, "group filter launch");
-    if ((e = launch_finish(p.block_size, ft, finish_wg, false, s)) != hipSuccess)
+    e = h->tiled ? launch_wnnm_tiles(wt, wnnm_wg, h->tile_lds, h->ncsr, s) : launch_wnnm(wt, wnnm_wg, h->ncsr, s);
+    if (e != hipSuccess) return hip_fail(e, "group filter launch");
+    if ((e = launch_finish(p.block_size, ft, finish_wg, h->tiled, s)) != hipSuccess)
         return hip_fail(e, "group filter finish launch");
     return NSS_HIP_OK;
 }
