@@ -59,6 +59,16 @@ inline constexpr uint32_t kTaken = 0xffffffffu;
 inline constexpr uint32_t kNonFinite = 0x7f800000u;
 inline constexpr int kXcds = 8;
 
+// Calls f(integral_constant<0>) .. f(integral_constant<N - 1>).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
 // Block index such that each XCD (blockIdx % 8 on dispatch) covers a
 // contiguous range of logical blocks; a bijection on [0, gridDim.x).
 __device__ inline int xcd_block() {
@@ -766,24 +776,38 @@ __global__ __launch_bounds__(64) void match_wave_kernel(MatchTable tab) {
 // MFMA matcher (B = 8, G <= 32): the role of the reference's tensor-core
 // matcher (src/cuda/common/match.cu:1165-1620, spatial_match_tensor), built
 // for CDNA4. A workgroup of four waves takes a block of 4 x 4 references.
-// The union of their windows is staged in LDS as fp16 values
-// h = fp16((v - mu) 2^S), S the block's power-of-two scale (the largest
-// |v - mu| then sits in [2^12, 2^13)). Dot products of reference and
-// candidate patches run on
-// v_mfma_f32_16x16x32_f16 (16 references x 16 candidates of one row per
-// tile), giving d' = |h_r|^2 + |h_c|^2 - 2 h_r.h_c for every pair; wave w
-// takes the candidate rows w mod 4. Two passes over the tiles:
-//   A. per reference, the four smallest upper bounds U of each lane's
-//      candidate column (16 lanes hold disjoint columns): the K-th smallest
-//      of those 64 distinct candidates bounds the K-th exact key from above;
+// The union of their windows is staged in LDS in FP32 (when that leaves four
+// workgroups per CU) and as fp16 values h = fp16((v - mu) 2^S), S a scale of
+// the block that keeps them below 2^13. Dot products of reference and
+// candidate patches run on v_mfma_f32_16x16x32_f16 (16 references x 16
+// candidates of one row per tile), giving d' = |h_r|^2 + |h_c|^2 - 2 h_r.h_c
+// for every pair; wave w takes the candidate rows w mod 4. A third MFMA adds
+// the candidates' norms with the bound's slope, and the accumulators start at
+// the reference's constant, +inf outside its window: the VALU sees finished
+// bounds, one operation per pair and pass. Two passes over the tiles:
+//   A. per reference, the smallest upper bound U of each of 64 classes of
+//      candidates (a lane's column residue, a wave's rows): the (K + 1)-th
+//      smallest of those (the reference itself is among them) bounds the K-th
+//      exact key from above;
 //   B. every candidate whose lower bound L does not exceed it is listed (at
-//      most 128 per reference for G <= 16, 256 for G <= 32).
+//      most 128 per reference for G <= 16, 192 for G <= 32), from the sign bits
+//      of L minus the bound.
 // The listed candidates are then scored in the FP32 order of the other
-// matchers (rows, then columns, one fmaf per pixel) and ranked by
+// matchers (rows, then columns, one fmaf per pixel) and taken in order of
 // (dist, y, x): the records are those of match_run_kernel bit for bit. A
 // reference whose list overflows, or a block holding a value fp16 cannot
-// carry (non-finite, or |v - mu| >= 8192 so that S would be negative),
-// scores its whole window exactly.
+// carry (non-finite, or |v - mu| >= 8192 so that S would be negative) or
+// nothing but one value, scores its whole window exactly.
+//
+// What bounds it: VALU issue (per wave of the step-3, range-16, group-16
+// launch 3.8 k instructions before the row scoring against 6.0 k with the
+// norms, masks and rank sums on the VALU) and LDS reads of the scoring. Per
+// 1080p YUV420 frame at step 3, range 16: group 16 on the noisy planes 660 us
+// (1115 before the norms and masks went into the MFMAs, the sums of ranks into
+// row minima and the reference's patch into registers), group 32 on the
+// denoised ones 1060 us (1758); gray 1080p, step 8, range 30, group 16: 258 us
+// (468). Lists of 160 cost 1340 us at group 32 (overflows), of 256 1126 (LDS:
+// four workgroups per CU instead of five).
 //
 // Error bound, in the scaled units (every distance times 2^2S; u = 2^-24):
 //   per element, |(v - mu) 2^S - h| <= 2^-11 |h| (1 + 2^-11) for a normal h,
@@ -796,7 +820,7 @@ __global__ __launch_bounds__(64) void match_wave_kernel(MatchTable tab) {
 //     sqrt(d''), d* the real SSD; with (a + b)^2 <= (1 + t) a^2 +
 //     (1 + 1/t) b^2, (a - b)^2 >= (1 - t) a^2 - (1/t - 1) b^2 (t = 2^-6)
 //     and E^2 <= 2 E_r^2 + 2 E_c^2 both bounds are linear in (c, |h_c|^2),
-//     c = |h_r|^2 - 2 h_r.h_c the MFMA tile: one FMA per pair;
+//     c = |h_r|^2 - 2 h_r.h_c the fp16 products' sum;
 //   the FP32 key differs from d* by at most 66 u d* (taken as 1e-4).
 // ---------------------------------------------------------------------------
 
@@ -804,9 +828,10 @@ typedef _Float16 mm_h16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 mm_h16x2 __attribute__((ext_vector_type(2)));
 typedef float mm_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t mm_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t mm_u32x2 __attribute__((ext_vector_type(2)));
+typedef float mm_f32x2 __attribute__((ext_vector_type(2)));
 
 inline constexpr float kMmC1 = 3.0517578125e-05f;    // 512 * 2^-24
-inline constexpr float kMmTiny = 6.103515625e-05f;   // 2^-14, fp16's smallest normal
 inline constexpr float kMmInf = __builtin_inff();
 inline constexpr float kMmT = 0.015625f;              // t = 2^-6
 inline constexpr float kMmKappa = 2.3889e-07f;        // 1.002 * 2^-22, rounded up
@@ -817,10 +842,9 @@ inline constexpr float kMmGammaL = 2.f * kMmKappa / kMmT;                // E^2 
 inline constexpr float kMmSlopeU = 1.f + kMmC1 + kMmGammaU / (1.f + kMmT) + 1e-6f;
 inline constexpr float kMmSlopeL = 1.f - kMmC1 - kMmGammaL / (1.f - kMmT) - 1e-6f;
 
-// fp16 bits of a scaled value (0 below 2^-14).
-__device__ inline uint32_t mm_half(float a) {
-    const _Float16 h = fabsf(a) < kMmTiny ? static_cast<_Float16>(0.f) : static_cast<_Float16>(a);
-    return __builtin_bit_cast(uint16_t, h);
+// Two fp16 values of one region word (rounded to nearest even).
+__device__ inline uint32_t mm_pack(float a, float b) {
+    return __builtin_bit_cast(uint32_t, mm_h16x2{static_cast<_Float16>(a), static_cast<_Float16>(b)});
 }
 
 // Eight fp16 values at region row `row`, columns col .. col + 7 (two per
@@ -852,16 +876,15 @@ __device__ inline float mm_rows_sum(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
-__device__ inline float wave_max_f32(float v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
-}
-
 // v of the lane DPP control CTRL selects (controls that stay inside a row).
 template <int CTRL>
 __device__ inline float dpp_f32(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
+template <int CTRL>
+__device__ inline uint32_t dpp_row_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xf, 0xf, true));
 }
 
 // The value of lane l (uniform).
@@ -888,27 +911,72 @@ __device__ inline float wave_max_dpp(float v) {
     return fmaxf(fmaxf(lane_f32(v, 0), lane_f32(v, 16)), fmaxf(lane_f32(v, 32), lane_f32(v, 48)));
 }
 
-// The FP32 key of the other matchers for B = 8: rows, then columns, one fmaf
-// per pixel.
-__device__ inline uint32_t mm_exact(const float* plane, size_t stride, int rx, int ry, int x, int y) {
-    const float* a = plane + static_cast<size_t>(ry) * stride + rx;
-    const float* b = plane + static_cast<size_t>(y) * stride + x;
+// Lane N's value of each 16-lane row, in all its lanes (row_newbcast).
+template <int N>
+__device__ __forceinline__ float row_bcast_f32(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, false));
+}
+
+// The FP32 key of the other matchers for B = 8 (rows, then columns, one fmaf
+// per pixel) with the reference's patch held by the 16-lane row (pixel 4 n + i
+// in lane n's patch[i]); b the candidate's first pixel, rows p apart. All 64
+// lanes must call. The broadcasts are operands of the subtractions, and only
+// the candidate is read: half the LDS words of reading both, which bound it.
+template <class Pitch>
+__device__ __forceinline__ uint32_t mm_exact_row(const float (&patch)[4], const float* b, Pitch p) {
     float acc = 0.f;
-    for (int py = 0; py < 8; ++py) {
+    static_for<8>([&](auto yc) {
+        constexpr int py = decltype(yc)::value;
+        float v[8];
 #pragma unroll
-        for (int px = 0; px < 8; ++px) {
-            const float d = a[py * stride + px] - b[py * stride + px];
+        for (int px = 0; px < 8; ++px) v[px] = b[py * p + px];
+        static_for<8>([&](auto xc) {
+            constexpr int px = decltype(xc)::value;
+            const float d = row_bcast_f32<2 * py + (px >> 2)>(patch[px & 3]) - v[px];
             acc = fmaf(d, d, acc);
-        }
-    }
+        });
+    });
     return dist_key(acc);
+}
+
+// Largest of the four 16-lane rows' values (each row's lanes hold the same).
+__device__ inline int wave_rows_max(int v) {
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// Minimum over the 16 lanes of each DPP row, returned to every lane of the
+// row (quad_perm, row_half_mirror, row_mirror: folded into the minima).
+__device__ inline uint32_t row_min_u32(uint32_t v) {
+    v = min(v, dpp_row_u32<0xb1>(v));
+    v = min(v, dpp_row_u32<0x4e>(v));
+    v = min(v, dpp_row_u32<0x141>(v));
+    return min(v, dpp_row_u32<0x140>(v));
+}
+
+// Minimum over the wave, uniform. All 64 lanes must call.
+__device__ inline uint32_t wave_min_u32_dpp(uint32_t v) {
+    v = row_min_u32(v);
+    const auto of = [&](int l) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), l)); };
+    return min(min(of(0), of(16)), min(of(32), of(48)));
+}
+
+// Whether a 16-bit field of m has two bits set or more.
+__device__ inline bool rows_with_two(unsigned long long m) {
+    bool two = false;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint32_t f = static_cast<uint32_t>(m >> (16 * r)) & 0xffffu;
+        two = two || (f & (f - 1u)) != 0u;
+    }
+    return two;
 }
 
 // Region row pitch in words: the smallest p >= 8 nt + 5 (16 nt + 8 halves
 // and the fifth word of an odd-column read) at which the four 16-lane rows
 // of a fragment read (each within 9 consecutive words, rows p apart) fall on
 // disjoint banks, for 32 banks (two rows per half-wave) and for 64.
-__host__ __device__ inline int mm_pitch(int nt) {
+constexpr int mm_pitch_of(int nt) {
     for (int p = 8 * nt + 5;; ++p) {
         const int a = p % 32;
         if (a < 9 || a > 23) continue;
@@ -922,6 +990,17 @@ __host__ __device__ inline int mm_pitch(int nt) {
         if (ok) return p;  // p = 16 mod 64 always qualifies
     }
 }
+inline constexpr int kMmTiles = 10;  // tile columns of the largest union (step 8, range 64)
+struct MmPitches {
+    int of[kMmTiles + 1];
+};
+constexpr MmPitches mm_pitches() {
+    MmPitches t{};
+    for (int i = 1; i <= kMmTiles; ++i) t.of[i] = mm_pitch_of(i);
+    return t;
+}
+__device__ constexpr MmPitches d_mm_pitch = mm_pitches();
+inline constexpr MmPitches h_mm_pitch = mm_pitches();
 
 struct MmWin {
     int cx, cy, left, right, top, bottom;
@@ -938,38 +1017,33 @@ __device__ inline MmWin mm_win(const MatchJob& jb, int i, int j) {
     return w;
 }
 
-// Minimum over the 16 lanes of each DPP row (rotations by 8, 4, 2, 1),
-// returned to every lane of the row.
-__device__ inline float row_min_f32(float v) {
-    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false)));
-    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false)));
-    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false)));
-    return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false)));
+__device__ inline uint32_t row_max_u32(uint32_t v) {
+    v = max(v, dpp_row_u32<0xb1>(v));
+    v = max(v, dpp_row_u32<0x4e>(v));
+    v = max(v, dpp_row_u32<0x141>(v));
+    return max(v, dpp_row_u32<0x140>(v));
 }
 
-// d into the ascending four s (the largest of the five dropped).
-__device__ inline void top4_insert(float (&s)[4], float d) {
-    // top down, so that each entry is overwritten after its last use
-    s[3] = __builtin_amdgcn_fmed3f(s[2], s[3], d);
-    s[2] = __builtin_amdgcn_fmed3f(s[1], s[2], d);
-    s[1] = __builtin_amdgcn_fmed3f(s[0], s[1], d);
-    s[0] = fminf(s[0], d);
-}
+// Pitch of the staged FP32 region for nt tile columns: its 16 nt + 8 columns,
+// and rows that start on different banks.
+__host__ __device__ constexpr int mm_pitch32(int nt) { return 16 * nt + 10; }
 
-// bf16 bits of v rounded towards +inf (an upper bound survives the exchange).
-__device__ inline uint16_t bf16_up(float v) {
-    const uint32_t b = __float_as_uint(v);
-    const uint32_t hi = b >> 16;
-    return static_cast<uint16_t>(((b & 0xffffu) != 0u && (b >> 31) == 0u) ? hi + 1u : hi);
-}
+inline constexpr int kMmCounters = 48;  // words of the counters, K values and bounds
 
-// LIST: listed candidates per reference (128 for G <= 16, 256 for G <= 32).
-template <int LIST>
-__global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
+// LIST: listed candidates per reference (128 for G <= 16, 192 for G <= 32).
+// STAGED: the FP32 region is held in LDS too, read from memory once (straight
+// to LDS); the scaling pass, the fp16 values and the exact keys come from it.
+// Without it (regions too large) those read the plane.
+template <int LIST, bool STAGED>
+__global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
     extern __shared__ __align__(16) uint32_t mm_lds[];
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: row loops branch on scalars
-    const int lb = xcd_block();
+    // Dispatch order, XCDs in turn: blocks cost what their content makes them
+    // list, and an XCD's own band of the frame would leave the others waiting
+    // (a band per XCD: 698 against 665 us on 1080p YUV420 at step 3, range 16,
+    // group 16); the regions' overlap is read from the last-level cache.
+    const int lb = static_cast<int>(blockIdx.x);
     const MatchJob& jb = tab.job[find_job(tab, lb)];
     const int blk = lb - jb.wg_begin;
     const int nbx = (jb.grid.nx + 3) >> 2;
@@ -985,20 +1059,20 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
     const int nt = (ux1 - ux0 + 16) >> 4;
     const int UW = 16 * nt;
     const int RH = uy1 - uy0 + 8;
-    const int pitch = mm_pitch(nt);
-    const int reg_words = max(RH * pitch, 16 * LIST);
+    const int pitch = d_mm_pitch.of[nt];
+    const int reg_words = (max(RH * pitch, 16 * LIST) + 3) & ~3;
     uint32_t* reg = mm_lds;
     // One area serves, in turn, the staging reductions and the pass-A
     // exchange (xw), the candidate lists (pass B, ranking), and the
     // fallback's keys.
-    constexpr int kUnion = 8 * LIST > 2048 ? 8 * LIST : 2048;           // words
+    constexpr int kUnion = 8 * LIST;                                    // words (at least the exchange's 1024)
     uint32_t* xw = mm_lds + reg_words;
-    uint16_t* xch = reinterpret_cast<uint16_t*>(xw);                    // [wave][j][lane][4] bf16
+    const int P32 = mm_pitch32(nt);
+    float* f32 = reinterpret_cast<float*>(mm_lds + reg_words + kUnion + kMmCounters);  // STAGED: rows of P32 floats
     uint16_t* list = reinterpret_cast<uint16_t*>(xw);                   // [16][LIST]
     int* cnt = reinterpret_cast<int*>(mm_lds + reg_words + kUnion);     // 16
-    int* pre = cnt + 16;                                                // 17 (+1 keeps 8-byte alignment)
-    int* kmv = pre + 18;                                                // 16
-    float* wl = reinterpret_cast<float*>(kmv + 16);                     // 16
+    int* kmv = cnt + 16;                                                // 16
+    float* wl = reinterpret_cast<float*>(kmv + 16);                     // 16 (kMmCounters words in all)
 
     // Per-reference counts K = min(G - 1, window - 1); counters cleared.
     if (tid < 16) {
@@ -1013,67 +1087,88 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
     }
 
     // mu: the mean of the first reference's patch (every wave alike). Two
-    // passes over the region, eight words per thread in flight each: the
-    // largest |v - mu| (non-finite values make it NaN), then the scaled
-    // fp16 values.
-    const float mu =
-        wave_sum_f32(plane[static_cast<size_t>(w00.cy + (lane >> 3)) * stride + w00.cx + (lane & 7)]) *
-        (1.f / 64.f);
-    const float inv_pitch = 1.f / static_cast<float>(pitch);
-    const int words = RH * pitch;
-    auto load8 = [&](int base, float (&v0)[8], float (&v1)[8]) {
+    // passes over the region: the largest |v - mu| as bits (a non-finite
+    // value's are the largest), then the scaled fp16 values. A wave's lanes
+    // take words_per consecutive words of rows_per rows (a whole row per
+    // step when a row has more than 64).
+    float mu;
+    const int wpr = 8 * nt + 4;  // words of a row that the fragments read
+    const int rows_per = wpr <= 64 ? 64 / wpr : 1;
+    const int lr = wpr <= 64 ? div_small(lane, 1.f / static_cast<float>(wpr)) : 0;
+    const int lw = wpr <= 64 ? lane - lr * wpr : lane;
+    // f(row, word, pixel, next pixel) of the region's words, four rows' loads
+    // in flight
+    auto each_word = [&](auto f) {
+        if (lr >= rows_per) return;
+        for (int w0 = lw; w0 < wpr; w0 += 64)
+            for (int y0 = wave * rows_per + lr; y0 < RH; y0 += 16 * rows_per) {
+                mm_f32x2 v[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int wd = base + tid + 256 * i;
-            v0[i] = mu;
-            v1[i] = mu;
-            if (wd < words) {
-                const int yy = div_small(wd, inv_pitch), xw2 = wd - yy * pitch;
-                const float* row = plane + static_cast<size_t>(uy0 + yy) * stride;
-                const int x = ux0 + 2 * xw2;
-                if (x < jb.width) v0[i] = row[x];
-                if (x + 1 < jb.width) v1[i] = row[x + 1];
+                for (int i = 0; i < 4; ++i) {
+                    const int yy = min(y0 + 4 * i * rows_per, RH - 1);
+                    if constexpr (STAGED) {
+                        v[i] = *reinterpret_cast<const mm_f32x2*>(f32 + yy * P32 + 2 * w0);
+                    } else {
+                        const float* row = plane + static_cast<size_t>(uy0 + yy) * stride;
+                        v[i][0] = row[min(ux0 + 2 * w0, jb.width - 1)];
+                        v[i][1] = row[min(ux0 + 2 * w0 + 1, jb.width - 1)];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (y0 + 4 * i * rows_per < RH) f(y0 + 4 * i * rows_per, w0, v[i][0], v[i][1]);
             }
-        }
     };
-    float amax = fabsf(mu - mu);  // NaN when mu is
-    for (int base = 0; base < words; base += 8 * 256) {
-        float v0[8], v1[8];
-        load8(base, v0, v1);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float a = fabsf(v0[i] - mu), b = fabsf(v1[i] - mu);
-            amax = (a > amax || a != a) ? a : amax;
-            amax = (b > amax || b != b) ? b : amax;
-        }
-    }
-    {
-        const float wm = wave_max_f32(amax);
-        const bool wn = __builtin_amdgcn_ballot_w64(amax != amax) != 0;
-        if (lane == 0) {
-            reinterpret_cast<float*>(xw)[wave] = wm;
-            xw[4 + wave] = wn ? 1u : 0u;
-        }
-    }
-    __syncthreads();
-    const float bmax = fmaxf(fmaxf(reinterpret_cast<float*>(xw)[0], reinterpret_cast<float*>(xw)[1]),
-                             fmaxf(reinterpret_cast<float*>(xw)[2], reinterpret_cast<float*>(xw)[3]));
-    // bmax < 2^e: S = 13 - e puts it below 2^13 (|-2 h| < 2^15 fits fp16)
-    int ex = 0;
-    (void)frexpf(bmax, &ex);
-    const int S = bmax > 0.f ? min(13 - ex, 40) : 40;
-    const bool anybad = (xw[4] | xw[5] | xw[6] | xw[7]) != 0u || !(bmax < 8192.f) || S < 0;
-    __syncthreads();
-    if (!anybad) {
-        const float sc = ldexpf(1.f, S);
-        for (int base = 0; base < words; base += 8 * 256) {
-            float v0[8], v1[8];
-            load8(base, v0, v1);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int wd = base + tid + 256 * i;
-                if (wd < words) reg[wd] = mm_half((v0[i] - mu) * sc) | (mm_half((v1[i] - mu) * sc) << 16);
+    if constexpr (STAGED) {
+        // Rows wave, wave + 4, ... by 64-column strips, each load straight to
+        // LDS (lane l's word lands at the wave-uniform address + 4 l); columns
+        // past the plane repeat its last (only masked candidates read them).
+        for (int c0 = 0; c0 < 16 * nt + 8; c0 += 64) {
+            const int xx = c0 + lane;
+            if (xx < 16 * nt + 8) {
+                const int gx = min(ux0 + xx, jb.width - 1);
+                for (int yy = wave; yy < RH; yy += 4)
+                    __builtin_amdgcn_global_load_lds(
+                        (const __attribute__((address_space(1))) void*)(plane + static_cast<size_t>(uy0 + yy) * stride + gx),
+                        (__attribute__((address_space(3))) void*)(f32 + yy * P32 + c0), 4, 0, 0);
             }
+        }
+        __syncthreads();
+        mu = wave_sum_dpp(f32[(w00.cy - uy0 + (lane >> 3)) * P32 + w00.cx - ux0 + (lane & 7)]) * (1.f / 64.f);
+    } else {
+        mu = wave_sum_dpp(plane[static_cast<size_t>(w00.cy + (lane >> 3)) * stride + w00.cx + (lane & 7)]) * (1.f / 64.f);
+    }
+    // S = 12 serves a largest |v - mu| in [2^-6, 2) (planes in [0, 1] with
+    // any structure): the first pass converts with it and finds the largest.
+    // Others convert again with their own S = 13 - e, bmax < 2^e: below 2^13
+    // either way (|-2 h| < 2^15 fits fp16).
+    // (v - mu) 2^S in one rounding: mu 2^S is exact. A value below fp16's
+    // smallest normal keeps an error below 2^-14 whether the products take it
+    // as a denormal or as 0.
+    uint32_t amax = __float_as_uint(mu) & 0x7fffffffu;
+    amax = amax >= kNonFinite ? amax : 0u;
+    each_word([&](int yy, int w, float v0, float v1) {
+        const float a0 = fmaf(v0, 4096.f, -mu * 4096.f), a1 = fmaf(v1, 4096.f, -mu * 4096.f);
+        amax = max(amax, __float_as_uint(a0) & 0x7fffffffu);
+        amax = max(amax, __float_as_uint(a1) & 0x7fffffffu);
+        reg[yy * pitch + w] = mm_pack(a0, a1);
+    });
+    amax = row_max_u32(amax);
+    if (n == 0) xw[wave * 4 + g] = amax;
+    __syncthreads();
+    const uint32_t bmax_bits = __builtin_amdgcn_readfirstlane(row_max_u32(xw[n]));
+    const float bmax = __uint_as_float(bmax_bits) * (1.f / 4096.f);
+    bool anybad = bmax_bits >= kNonFinite || !(bmax < 8192.f);
+    if (!anybad && !(bmax >= 0.015625f && bmax < 2.f)) {
+        int ex = 0;
+        (void)frexpf(bmax, &ex);
+        const int S = min(13 - ex, 40);
+        anybad = S < 0 || bmax == 0.f;  // a constant region: every candidate would be listed
+        if (!anybad) {
+            const float sc = ldexpf(1.f, S), msc = -mu * sc;
+            each_word([&](int yy, int w, float v0, float v1) {
+                reg[yy * pitch + w] = mm_pack(fmaf(v0, sc, msc), fmaf(v1, sc, msc));
+            });
         }
     }
     __syncthreads();
@@ -1095,143 +1190,141 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
         A1 *= static_cast<_Float16>(-2.f);
         // C layout: lane (g, n) holds references 4 g + j (column g, row j)
         // against candidate n of the tile.
-        mm_f32x4 nr;
+        float nr[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) nr[j] = __shfl(nrA, 4 * g + j, 64);
         const bool cval = g < ncol;
         const MmWin cw = mm_win(jb, i0 + min(g, ncol - 1), j0);
-        const int ccx = cw.cx, cleft = cval ? cw.left : (1 << 30), cright = cval ? cw.right : -1;
-        int rtop[4], rbot[4], rcy[4];
+        const int cleft = cval ? cw.left - ux0 : (1 << 30), cright = cval ? cw.right - ux0 : -1;
+        // Each wave takes the candidate rows uy0 + wave + 4 i, i < steps; row
+        // j's windows hold the steps i with i - first[j] <= count[j] (unsigned;
+        // uniform, so the tests below are scalar).
+        const int steps = (uy1 - uy0 - wave + 4) >> 2;
+        int first[4];
+        uint32_t count[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            // uniform: the row tests below branch on scalars
             const MmWin w = mm_win(jb, i0, j0 + min(j, nrow - 1));
-            rcy[j] = __builtin_amdgcn_readfirstlane(w.cy);
-            rtop[j] = __builtin_amdgcn_readfirstlane(j < nrow ? w.top : (1 << 30));
-            rbot[j] = __builtin_amdgcn_readfirstlane(j < nrow ? w.bottom : -1);
+            const int a = (max(w.top - uy0 - wave, 0) + 3) >> 2, b = (w.bottom - uy0 - wave) >> 2;
+            const bool any = j < nrow && w.bottom - uy0 - wave >= 0 && b >= a;
+            first[j] = __builtin_amdgcn_readfirstlane(any ? a : 1 << 30);
+            count[j] = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(any ? b - a : 0));
         }
+        auto holds = [&](int i, int j) { return static_cast<uint32_t>(i - first[j]) <= count[j]; };
 
-        // Each wave takes the candidate rows y = uy0 + wave (mod 4).
-        float s[4][4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int k = 0; k < 4; ++k) s[j][k] = kMmInf;
-        float wv[4] = {0.f, 0.f, 0.f, 0.f};
-        // One row step over NC tile columns at once: independent chains
-        // (fragment loads, norms, two MFMAs, epilogue) for the scheduler to
-        // interleave.
-        auto pass_cols = [&](auto surv_tag, auto nc_tag, int t0) {
-            constexpr bool SURV = decltype(surv_tag)::value;
+        // The tiles of NC tile columns from t0 on, row step by row step. A
+        // tile is three MFMAs on c0: slope |h_c|^2 (lane (g, n)'s rows g and
+        // g + 4 squared, summed over g by a row of slopes), then the two halves
+        // of -2 h_r.h_c. c0 is each reference's start value, +inf where the
+        // candidate column lies outside its window: no masks, norms or scaling
+        // are left for the VALU. use(i, c) sees step i's tiles.
+        auto pass_cols = [&](auto nc_tag, int t0, float slope, const float (&start)[4], auto use) {
             constexpr int NC = decltype(nc_tag)::value;
-            int col[NC];
-            bool xv[NC], xs[NC];
+            mm_f32x4 c0[NC];
+            mm_h16x8 F[2][NC];
+            float sq[2][NC];
 #pragma unroll
             for (int q = 0; q < NC; ++q) {
-                col[q] = 16 * (t0 + q) + n;
-                const int x = ux0 + col[q];
-                xv[q] = x >= cleft && x <= cright;
-                xs[q] = x == ccx;
-            }
-            int y = uy0 + wave;
-            if (y > uy1) return;
-            mm_h16x8 F0[NC];
-            float T0[NC];
+                const int col = 16 * (t0 + q) + n;
+                const bool in = col >= cleft && col <= cright;
 #pragma unroll
-            for (int q = 0; q < NC; ++q) {
-                F0[q] = mm_frag(reg, pitch, y - uy0 + g, col[q]);
-                T0[q] = mm_rows_sum(mm_sq(F0[q]));
+                for (int j = 0; j < 4; ++j) c0[q][j] = in ? start[j] : kMmInf;
+                F[0][q] = mm_frag(reg, pitch, wave + g, col);
+                sq[0][q] = mm_sq(F[0][q]);
             }
-            for (; y <= uy1; y += 4) {
-                mm_h16x8 F1[NC];
-                float T1[NC];
+            auto step = [&](int i, const mm_h16x8 (&fa)[NC], const float (&sa)[NC], mm_h16x8 (&fb)[NC],
+                            float (&sb)[NC]) {
                 mm_f32x4 c[NC];
 #pragma unroll
                 for (int q = 0; q < NC; ++q) {
-                    F1[q] = mm_frag(reg, pitch, y - uy0 + 4 + g, col[q]);
-                    T1[q] = mm_rows_sum(mm_sq(F1[q]));
-                    c[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, F0[q], nr, 0, 0, 0);
-                    c[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, F1[q], c[q], 0, 0, 0);
+                    fb[q] = mm_frag(reg, pitch, wave + 4 * i + 4 + g, 16 * (t0 + q) + n);
+                    sb[q] = mm_sq(fb[q]);
+                    c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(slope, sa[q] + sb[q], c0[q], 0, 0, 0);
+                    c[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, fa[q], c[q], 0, 0, 0);
+                    c[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, fb[q], c[q], 0, 0, 0);
                 }
-#pragma unroll
-                for (int q = 0; q < NC; ++q) {
-                    const float ncx = xv[q] ? T0[q] + T1[q] : kMmInf;
-                    bool sv[4] = {false, false, false, false};
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // reference row j's window holds row y: uniform
-                        if (y >= rtop[j] && y <= rbot[j]) {
-                            // pass A: U / (1 + t) up to a per-reference
-                            // constant; pass B: L / (1 - t) likewise
-                            float d = fmaf(ncx, SURV ? kMmSlopeL : kMmSlopeU, c[q][j]);
-                            if (y == rcy[j]) d = xs[q] ? kMmInf : d;  // the reference itself
-                            if constexpr (SURV)
-                                sv[j] = d <= wv[j];
-                            else
-                                top4_insert(s[j], d);
-                        }
-                    }
-                    if constexpr (SURV) {
-                        if (__builtin_amdgcn_ballot_w64(sv[0] || sv[1] || sv[2] || sv[3]) != 0) {
-                            const int u = (y - uy0) * UW + col[q];
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) {
-                                if (sv[j]) {
-                                    const int m = 4 * g + j;
-                                    const int k = atomicAdd(&cnt[m], 1);
-                                    if (k < LIST) list[m * LIST + k] = static_cast<uint16_t>(u);
-                                }
-                            }
-                        }
-                    }
-                    F0[q] = F1[q];
-                    T0[q] = T1[q];
-                }
+                use(i, c);
+            };
+            for (int i = 0; i < steps; i += 2) {
+                step(i, F[0], sq[0], F[1], sq[1]);
+                if (i + 1 < steps) step(i + 1, F[1], sq[1], F[0], sq[0]);
             }
         };
-        auto pass = [&](auto surv_tag) {
-            int t = 0;
-            for (; t + 2 <= nt; t += 2) pass_cols(surv_tag, std::integral_constant<int, 2>{}, t);
-            if (t < nt) pass_cols(surv_tag, std::integral_constant<int, 1>{}, t);
+        auto pass = [&](float slope, const float (&start)[4], auto use) {
+            for (int t = 0; t < nt;) {
+                const int left = nt - t;
+                if (left == 3 || left > 4) {
+                    pass_cols(std::integral_constant<int, 3>{}, t, slope, start,
+                              [&](int i, const mm_f32x4 (&c)[3]) { use(std::integral_constant<int, 3>{}, t, i, c); });
+                    t += 3;
+                } else if (left >= 2) {
+                    pass_cols(std::integral_constant<int, 2>{}, t, slope, start,
+                              [&](int i, const mm_f32x4 (&c)[2]) { use(std::integral_constant<int, 2>{}, t, i, c); });
+                    t += 2;
+                } else {
+                    pass_cols(std::integral_constant<int, 1>{}, t, slope, start,
+                              [&](int i, const mm_f32x4 (&c)[1]) { use(std::integral_constant<int, 1>{}, t, i, c); });
+                    t += 1;
+                }
+            }
         };
 
-        pass(std::false_type{});
+        // Pass A: U / (1 + t) up to a per-reference constant; each lane keeps
+        // the smallest of its candidates per reference (the positions of one
+        // residue mod 16 columns and 4 rows: 64 disjoint classes). The start
+        // is raised by the bound's own C1 |h_r|^2, and 2^-4: d' + C1 (|h_r|^2 +
+        // |h_c|^2) stays above the sums' rounding, so the sums are positive,
+        // order as their bits do, and the minimum is an integer one.
+        float raised[4];
+        uint32_t s[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j) {
+            raised[j] = fmaf(nr[j], 1.f + kMmC1, 0.0625f);
+            s[j] = kNonFinite;
+        }
+        pass(kMmSlopeU, raised, [&](auto nc_tag, int, int i, const auto& c) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) xch[((wave * 4 + j) * 64 + lane) * 4 + k] = bf16_up(s[j][k]);
+            for (int j = 0; j < 4; ++j)
+                if (holds(i, j))
+#pragma unroll
+                    for (int q = 0; q < decltype(nc_tag)::value; ++q) s[j] = min(s[j], __float_as_uint(c[q][j]));
+        });
+        uint32_t* xch = xw;  // [wave][j][lane]
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xch[(wave * 4 + j) * 64 + lane] = s[j];
         __syncthreads();
-        // Wave w: references of row j = w. Each lane merges the four waves'
-        // four smallest of its candidate column; the K-th smallest over the
-        // row's 16 lanes (64 distinct candidates) by rounds of a row minimum.
+        // Wave w: references of row j = w. The (K + 1)-th smallest of the 64
+        // classes' minima (the reference itself is one of the candidates) by
+        // rounds of a row minimum over each lane's sorted four.
         {
-            float m4[4] = {kMmInf, kMmInf, kMmInf, kMmInf};
-            for (int v = 0; v < 4; ++v)
+            uint32_t m4[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    top4_insert(m4, __uint_as_float(static_cast<uint32_t>(xch[((v * 4 + wave) * 64 + lane) * 4 + k])
-                                                    << 16));
+            for (int v = 0; v < 4; ++v) m4[v] = xch[(v * 4 + wave) * 64 + lane];
+            auto order = [&](int a, int b) {
+                const uint32_t lo = min(m4[a], m4[b]), hi = max(m4[a], m4[b]);
+                m4[a] = lo;
+                m4[b] = hi;
+            };
+            order(0, 1), order(2, 3), order(0, 2), order(1, 3), order(1, 2);
             const int K = kmv[4 * g + wave];
             int taken = 0;
-            bool found = K == 0;
-            float td = kMmInf;
-            for (int round = 0; round < 32; ++round) {
-                if (__builtin_amdgcn_ballot_w64(!found) == 0) break;
-                const float mn = row_min_f32(m4[0]);
+            uint32_t tdb = kNonFinite;
+            bool open = K > 0;
+            while (__builtin_amdgcn_ballot_w64(open) != 0) {  // at most 64 / 16 + K rounds: each takes a class
+                const uint32_t mn = row_min_u32(m4[0]);
                 const bool eq = m4[0] == mn;
                 const unsigned long long bal = __builtin_amdgcn_ballot_w64(eq);
-                taken += __popcll((bal >> (16 * g)) & 0xffffull);
-                if (eq) {
-                    m4[0] = m4[1];
-                    m4[1] = m4[2];
-                    m4[2] = m4[3];
-                    m4[3] = kMmInf;
-                }
-                if (!found && taken >= K) {
-                    found = true;
-                    td = mn;
+                taken += __popc(static_cast<uint32_t>(bal >> (16 * g)) & 0xffffu);
+                m4[0] = eq ? m4[1] : m4[0];
+                m4[1] = eq ? m4[2] : m4[1];
+                m4[2] = eq ? m4[3] : m4[2];
+                m4[3] = eq ? kNonFinite : m4[3];
+                if (open && taken > K) {
+                    open = false;
+                    tdb = mn;
                 }
             }
+            const float td = __uint_as_float(tdb);
             if (n == 0) {
                 const float nrm = wave == 0 ? nr[0] : wave == 1 ? nr[1] : wave == 2 ? nr[2] : nr[3];
                 float wt = -kMmInf;
@@ -1242,7 +1335,8 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
                         // U = (1 + t) td + beta_U bounds the K-th key;
                         // a candidate survives while its L = (1 - t) v -
                         // beta_L does not exceed U.
-                        const float betaU = (1.f + kMmT) * kMmC1 * nrm + kMmGammaU * (nrm + 2.f);
+                        // (td holds C1 nrm already)
+                        const float betaU = kMmGammaU * (nrm + 2.f);
                         const float betaL = (1.f - kMmT) * kMmC1 * nrm + kMmGammaL * (nrm + 2.f);
                         const float U = ((1.f + kMmT) * td + betaU) * 1.0001f;
                         wt = (U * 1.0001f + betaL) / (1.f - kMmT) * 1.00001f;
@@ -1252,58 +1346,123 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
             }
         }
         __syncthreads();
+        // Pass B: L / (1 - t) likewise, started at minus the bound: a negative
+        // sum survives (equality too: the bound's own margins are far above a
+        // rounding). Its sign goes into the lane's word of the tile column,
+        // newest lowest; every eight steps, and at the end, the words' bits are
+        // listed.
+        float below[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) wv[j] = wl[4 * g + j];
-        pass(std::true_type{});
+        for (int j = 0; j < 4; ++j) below[j] = nr[j] - wl[4 * g + j];
+        uint32_t word[3] = {0u, 0u, 0u}, valid = 0u;
+        pass(kMmSlopeL, below, [&](auto nc_tag, int t, int i, const auto& c) {
+            constexpr int NC = decltype(nc_tag)::value;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                valid = (valid << 1) | (holds(i, j) ? 1u : 0u);
+#pragma unroll
+                for (int q = 0; q < NC; ++q) word[q] = __builtin_amdgcn_alignbit(word[q], __float_as_uint(c[q][j]), 31);
+            }
+            if ((i & 7) != 7 && i + 1 != steps) return;
+#pragma unroll
+            for (int q = 0; q < NC; ++q) {
+                uint32_t bits = word[q] & valid;
+                while (bits) {
+                    const int at = __builtin_ctz(bits);  // step i - at / 4, row j = 3 - at % 4
+                    bits &= bits - 1u;
+                    const int m = 4 * g + 3 - (at & 3);
+                    const int u = (wave + 4 * (i - (at >> 2))) * UW + 16 * (t + q) + n;
+                    const int k = atomicAdd(&cnt[m], 1);
+                    if (k < LIST) list[m * LIST + k] = static_cast<uint16_t>(u);
+                }
+            }
+            valid = 0u;
+        });
     }
     __syncthreads();
 
-    // Listed candidates: exact keys (into the region's words), then ranks.
-    if (tid == 0) {
-        int acc = 0;
-        for (int m = 0; m < 16; ++m) {
-            pre[m] = acc;
-            const int c = cnt[m];
-            acc += (!anybad && kmv[m] > 0 && c <= LIST) ? c : 0;
-        }
-        pre[16] = acc;
-    }
-    __syncthreads();
-    const int total = pre[16];
-    const float inv_uw = 1.f / static_cast<float>(UW);
-    uint32_t* dk = reg;
-    auto item = [&](int q, int& m, int& sl) {
-        m = 0;
+    // The patch at (x, y) over the lanes of a 16-lane row, and the exact key of
+    // such a patch against the one at region column ux, row uy.
+    auto row_patch = [&](int x, int y, float (&patch)[4]) {
 #pragma unroll
-        for (int b = 8; b >= 1; b >>= 1)
-            if (m + b < 16 && q >= pre[m + b]) m += b;
-        sl = q - pre[m];
-    };
-    for (int q = tid; q < total; q += 256) {
-        int m, sl;
-        item(q, m, sl);
-        const int u = list[m * LIST + sl];
-        const int uy = div_small(u, inv_uw), ux = u - uy * UW;
-        const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
-        dk[q] = mm_exact(plane, stride, w.cx, w.cy, ux0 + ux, uy0 + uy);
-    }
-    __syncthreads();
-    for (int q = tid; q < total; q += 256) {
-        int m, sl;
-        item(q, m, sl);
-        const int c = pre[m + 1] - pre[m];
-        const uint32_t d = dk[q];
-        const int u = list[m * LIST + sl];
-        int rank = 0;
-        for (int s2 = 0; s2 < c; ++s2) {
-            const uint32_t d2 = dk[pre[m] + s2];
-            const int u2 = list[m * LIST + s2];
-            rank += (d2 < d || (d2 == d && u2 < u)) ? 1 : 0;
+        for (int i = 0; i < 4; ++i) {
+            const int py = y + (n >> 1), px = x + 4 * (n & 1) + i;
+            patch[i] = STAGED ? f32[(py - uy0) * P32 + px - ux0] : plane[static_cast<size_t>(py) * stride + px];
         }
-        if (rank < kmv[m]) {
-            const int uy = div_small(u, inv_uw), ux = u - uy * UW;
-            const int ref_id = (j0 + (m & 3)) * jb.grid.nx + i0 + (m >> 2);
-            jb.out[static_cast<size_t>(ref_id) * G + 1 + rank] = MatchRec{ux0 + ux, uy0 + uy, jb.t0, d};
+    };
+    auto exact = [&](const float (&patch)[4], int ux, int uy) {
+        if constexpr (STAGED)
+            return mm_exact_row(patch, f32 + uy * P32 + ux, P32);
+        else
+            return mm_exact_row(patch, plane + static_cast<size_t>(uy0 + uy) * stride + ux0 + ux, stride);
+    };
+
+    // Listed candidates: lane n of row g of wave w scores the entries n,
+    // n + 16, ... of reference m = 4 w + g exactly, its patch spread over the
+    // row's lanes (four pixels each, broadcast by DPP), and keeps its four
+    // smallest by (distance, place). The records then come in order by rounds
+    // of a row minimum; all of it inside the wave, every lane active.
+    {
+        const int m = 4 * wave + g;
+        const int c0 = cnt[m];
+        const int c = (!anybad && kmv[m] > 0 && c0 <= LIST) ? c0 : 0, K = c > 0 ? kmv[m] : 0;
+        const int cmax = wave_rows_max(c), kmax = wave_rows_max(K);
+        const float inv_uw = 1.f / static_cast<float>(UW);
+        uint32_t* dk = reg + m * LIST;
+        const uint16_t* lm = list + m * LIST;
+        const int cx = ref_x(jb.grid, min(i0 + (m >> 2), jb.grid.nx - 1), jb.width, 8);
+        const int cy = ref_y(jb.grid, min(j0 + (m & 3), jb.grid.ny - 1), jb.height, 8);
+        const uint32_t self = (static_cast<uint32_t>(cy - uy0) << 16) | static_cast<uint32_t>(cx - ux0);
+        float patch[4];
+        row_patch(cx, cy, patch);
+        unsigned long long best[4] = {~0ull, ~0ull, ~0ull, ~0ull};
+        auto place = [&](int q) {  // region row and column of entry q, as one ordered word
+            const int u = lm[q];
+            const int uy = div_small(u, inv_uw);
+            return (static_cast<uint32_t>(uy) << 16) | static_cast<uint32_t>(u - uy * UW);
+        };
+        auto insert = [&](uint32_t d, uint32_t at) {
+            const unsigned long long x = (static_cast<unsigned long long>(d) << 32) | at;
+            best[3] = min(best[3], x);
+#pragma unroll
+            for (int k = 3; k > 0; --k) {
+                const unsigned long long lo = min(best[k], best[k - 1]), hi = max(best[k], best[k - 1]);
+                best[k - 1] = lo;
+                best[k] = hi;
+            }
+        };
+        for (int q0 = 0; q0 < cmax; q0 += 16) {
+            const int q = q0 + n;
+            const uint32_t at = q < c ? place(q) : self;
+            const int uy = static_cast<int>(at >> 16), ux = static_cast<int>(at & 0xffffu);
+            uint32_t d = exact(patch, ux, uy);
+            if (at == self) d = kTaken;  // listed with the rest, never taken
+            if (q < c) dk[q] = d;
+            insert(d, at);
+        }
+        MatchRec* out = jb.out + (static_cast<size_t>(j0 + (m & 3)) * jb.grid.nx + i0 + (m >> 2)) * G + 1;
+        int given = 0;
+        for (int k = 0; k < kmax; ++k) {
+            const uint32_t d = static_cast<uint32_t>(best[0] >> 32), at = static_cast<uint32_t>(best[0]);
+            const uint32_t mn = row_min_u32(d);
+            bool mine = d == mn && k < K;
+            const unsigned long long who = __builtin_amdgcn_ballot_w64(mine);
+            if (rows_with_two(who)) {  // equal distances: the first place
+                const uint32_t first = row_min_u32(mine ? at : ~0u);
+                mine = mine && at == first;
+            }
+            if (mine) {
+                out[k] = MatchRec{ux0 + static_cast<int>(at & 0xffffu), uy0 + static_cast<int>(at >> 16), jb.t0, d};
+                best[0] = best[1], best[1] = best[2], best[2] = best[3], best[3] = ~0ull;
+                if (++given == 4) {  // the lane's next four
+                    given = 0;
+                    const unsigned long long won = (static_cast<unsigned long long>(d) << 32) | at;
+                    for (int q = n; q < c; q += 16) {
+                        const unsigned long long x = (static_cast<unsigned long long>(dk[q]) << 32) | place(q);
+                        if (x > won && x < best[3]) insert(dk[q], static_cast<uint32_t>(x));
+                    }
+                }
+            }
         }
     }
     if (tid < 16 && (tid >> 2) < ncol && (tid & 3) < nrow) {
@@ -1313,59 +1472,143 @@ __global__ __launch_bounds__(256) void match_mfma_kernel(MatchTable tab) {
         jb.counts[ref_id] = 1 + kmv[tid];
     }
 
-    __syncthreads();  // the lists' area becomes the fallback's keys
-    // Whole windows, exactly, for the references the bound could not serve
-    // (wave w takes references w, w + 4, ...): chunks of 64 candidates merged
-    // by rank into the running G - 1 best.
-    unsigned long long* ck = reinterpret_cast<unsigned long long*>(xw) + wave * 128;  // 64
-    unsigned long long* bk = ck + 64;                                                  // 32
-    unsigned long long* nbk = bk + 32;                                                 // 32
-    for (int m = wave; m < 16; m += 4) {
-        const int K = kmv[m];
-        if (K == 0 || !(anybad || cnt[m] > LIST)) continue;
-        const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
-        const int ww = w.right - w.left + 1, ncand = ww * (w.bottom - w.top + 1);
-        const int self = (w.cy - w.top) * ww + (w.cx - w.left);
-        const float inv_ww = 1.f / static_cast<float>(ww);
-        int nb = 0;
-        for (int base = 0; base < ncand; base += 64) {
-            const int c = base + lane;
-            unsigned long long key = ~0ull;
-            if (c < ncand && c != self) {
+    // (no reference of the block needs the rest: the usual case)
+    if (__builtin_amdgcn_ballot_w64(kmv[n] > 0 && (anybad || cnt[n] > LIST)) == 0) return;
+    __syncthreads();  // the regions and lists become the fallback's keys
+    // Whole windows, exactly, for the references the bound could not serve:
+    // up to four at a time, the workgroup scores each window's candidates (one
+    // per thread) into LDS, then a wave per reference takes the G - 1 smallest
+    // by rounds of a wave minimum over each lane's four best. Windows that do
+    // not fit come in pieces; the lanes carry the best so far. A window whose
+    // first 256 places hold G - 1 copies of the patch (distance 0) is done with
+    // those: no later place can displace one (flat areas).
+    const int space = reg_words + kUnion;
+    const int wcap = min((2 * jb.range + 1) * (2 * jb.range + 1), (ux1 - ux0 + 1) * (uy1 - uy0 + 1));
+    const int at_once = max(1, min(4, space / wcap));
+    const int piece = min(wcap, space);
+    int* copies = reinterpret_cast<int*>(wl);  // per reference at work
+    uint32_t todo = static_cast<uint32_t>(
+        __builtin_amdgcn_ballot_w64(kmv[n] > 0 && (anybad || cnt[n] > LIST)) & 0xffffull);
+    while (todo) {
+        uint32_t refs = 0u;  // a reference per nibble
+        int nref = 0;
+        for (; nref < at_once && todo; ++nref, todo &= todo - 1u)
+            refs |= static_cast<uint32_t>(__builtin_ctz(todo)) << (4 * nref);
+        if (tid < 4) copies[tid] = 0;
+        __syncthreads();
+        unsigned long long kept = ~0ull;  // lane k: the k-th best of the pieces so far
+        uint32_t flat = 0u;               // the references done after 256 places, a bit each
+        // keys of places from .. to - 1 (p0 the piece's first) of the r-th reference
+        auto score = [&](int r, int p0, int from, int to) {
+            const int m = (refs >> (4 * r)) & 15;
+            const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
+            const int ww = w.right - w.left + 1, end = min(ww * (w.bottom - w.top + 1), to);
+            const int self = (w.cy - w.top) * ww + (w.cx - w.left);
+            const float inv_ww = 1.f / static_cast<float>(ww);
+            float patch[4];
+            row_patch(w.cx, w.cy, patch);
+            int zeros = 0;
+            for (int q0 = from + 64 * wave; q0 < end; q0 += 256) {
+                const int c = min(q0 + lane, end - 1);
                 const int dy = div_small(c, inv_ww), dx = c - dy * ww;
-                key = (static_cast<unsigned long long>(mm_exact(plane, stride, w.cx, w.cy, w.left + dx, w.top + dy))
-                       << 32) |
-                      static_cast<uint32_t>(c);
+                const uint32_t d = exact(patch, w.left - ux0 + dx, w.top - uy0 + dy);
+                mm_lds[r * piece + c - p0] = c == self ? kTaken : d;
+                zeros += __popcll(__builtin_amdgcn_ballot_w64(d == 0u && c != self && q0 + lane < end));
             }
-            ck[lane] = key;
-            wave_sync();
-            int rank = 0, brank = 0;
-            unsigned long long bkey = ~0ull;
-            for (int q = 0; q < 64; ++q) rank += ck[q] < key ? 1 : 0;
-            for (int j = 0; j < nb; ++j) rank += bk[j] < key ? 1 : 0;
-            if (lane < nb) {
-                bkey = bk[lane];
-                brank = lane;
-                for (int q = 0; q < 64; ++q) brank += ck[q] < bkey ? 1 : 0;
-            }
-            const int nvalid = __popcll(__builtin_amdgcn_ballot_w64(key != ~0ull));
-            wave_sync();
-            if (key != ~0ull && rank < K) nbk[rank] = key;
-            if (lane < nb && brank < K) nbk[brank] = bkey;
-            nb = min(K, nb + nvalid);
-            wave_sync();
-            if (lane < nb) bk[lane] = nbk[lane];
-            wave_sync();
-        }
-        if (lane < K) {
-            const unsigned long long key = bk[lane];
-            const int c = static_cast<int>(static_cast<uint32_t>(key));
-            const int dy = div_small(c, inv_ww), dx = c - dy * ww;
-            const int ref_id = (j0 + (m & 3)) * jb.grid.nx + i0 + (m >> 2);
-            jb.out[static_cast<size_t>(ref_id) * G + 1 + lane] =
+            return zeros;
+        };
+        // record k of reference m: a key (distance, place in the window)
+        auto store = [&](int m, int k, unsigned long long key) {
+            const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
+            const int ww = w.right - w.left + 1, c = static_cast<int>(static_cast<uint32_t>(key));
+            const int dy = div_small(c, 1.f / static_cast<float>(ww)), dx = c - dy * ww;
+            jb.out[(static_cast<size_t>(j0 + (m & 3)) * jb.grid.nx + i0 + (m >> 2)) * G + 1 + k] =
                 MatchRec{w.left + dx, w.top + dy, jb.t0, static_cast<uint32_t>(key >> 32)};
+        };
+        for (int p0 = 0; p0 < wcap && flat != (1u << nref) - 1u; p0 += piece) {
+            int from = p0;
+            if (p0 == 0) {
+                from = min(piece, 256);
+                for (int r = 0; r < nref; ++r) {
+                    const int zeros = score(r, 0, 0, from);
+                    if (lane == 0) atomicAdd(&copies[r], zeros);
+                }
+                __syncthreads();
+                for (int r = 0; r < nref; ++r)
+                    flat |= copies[r] >= kmv[(refs >> (4 * r)) & 15] ? 1u << r : 0u;
+            }
+            const uint32_t skip = __builtin_amdgcn_readfirstlane(flat);
+            for (int r = 0; r < nref; ++r)
+                if (!((skip >> r) & 1u)) score(r, p0, from, p0 + piece);
+            __syncthreads();
+            const bool copied = (skip >> wave) & 1u;
+            const int m = wave < nref ? (refs >> (4 * wave)) & 15 : 0;
+            const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
+            const int last = min((w.right - w.left + 1) * (w.bottom - w.top + 1), copied ? from : p0 + piece) - p0;
+            const uint32_t* keys = mm_lds + wave * piece;
+            const int K = wave < nref ? kmv[m] : 0;
+            if (copied) {  // the first K copies, in order
+                int rank = 0;
+                for (int c0 = 0; p0 == 0 && c0 < last && rank < K; c0 += 64) {
+                    const bool zero = c0 + lane < last && keys[min(c0 + lane, last - 1)] == 0u;
+                    const unsigned long long z = __builtin_amdgcn_ballot_w64(zero);
+                    const int k = rank + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(z >> 32),
+                                                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(z), 0u));
+                    if (zero && k < K) store(m, k, static_cast<unsigned long long>(c0 + lane));
+                    rank += __popcll(z);
+                }
+            } else if (wave < nref) {
+                const unsigned long long carried = lane < K ? kept : ~0ull;
+                unsigned long long best[4];
+                auto insert = [&](unsigned long long x) {
+                    best[3] = x;
+#pragma unroll
+                    for (int k = 3; k > 0; --k)
+                        if (best[k] < best[k - 1]) {
+                            const unsigned long long t = best[k];
+                            best[k] = best[k - 1];
+                            best[k - 1] = t;
+                        }
+                };
+                // the lane's four smallest keys from `from` on
+                auto collect = [&](unsigned long long from) {
+                    best[0] = best[1] = best[2] = best[3] = ~0ull;
+                    if (carried >= from) insert(carried);
+                    for (int c = lane; c < last; c += 64) {
+                        const uint32_t d = keys[c];
+                        const unsigned long long x = (static_cast<unsigned long long>(d) << 32) | static_cast<uint32_t>(p0 + c);
+                        if (d != kTaken && x >= from && x < best[3]) insert(x);
+                    }
+                };
+                collect(0ull);
+                int given = 0;
+                for (int k = 0; k < K; ++k) {
+                    const uint32_t d = static_cast<uint32_t>(best[0] >> 32), at = static_cast<uint32_t>(best[0]);
+                    const uint32_t mn = wave_min_u32_dpp(d);
+                    bool mine = d == mn;
+                    const unsigned long long who = __builtin_amdgcn_ballot_w64(mine);
+                    uint32_t first = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), __builtin_ctzll(who)));
+                    if ((who & (who - 1u)) != 0) {  // equal distances: the first place
+                        first = wave_min_u32_dpp(mine ? at : ~0u);
+                        mine = mine && at == first;
+                    }
+                    const unsigned long long win = (static_cast<unsigned long long>(mn) << 32) | first;
+                    if (lane == k) kept = win;
+                    if (mine && win != ~0ull) {
+                        best[0] = best[1], best[1] = best[2], best[2] = best[3], best[3] = ~0ull;
+                        if (++given == 4) {
+                            given = 0;
+                            collect(win + 1u);
+                        }
+                    }
+                }
+            }
+            __syncthreads();
         }
-        wave_sync();
+        if (wave < nref && !((flat >> wave) & 1u)) {
+            const int m = (refs >> (4 * wave)) & 15;
+            if (lane < kmv[m]) store(m, lane, kept);
+        }
     }
 }
 
@@ -3993,16 +4236,6 @@ __global__ __launch_bounds__(64) void ncsr_group_kernel(WnnmTable tab) {
 // waits a third of its cycles.
 // ---------------------------------------------------------------------------
 
-// Calls f(integral_constant<0>) .. f(integral_constant<N - 1>).
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // rr_partner for a full group.
 template <int N>
 __host__ __device__ constexpr int rr_pair(int i, int r) {
@@ -4386,20 +4619,34 @@ size_t match_wave_lds_bytes(int block, int range, bool stage) {
     return ((reg + 3) & ~static_cast<size_t>(3)) * 4 + cand;
 }
 
-static int mm_list(int group) { return group > 16 ? 256 : 128; }
+static int mm_list(int group) { return group > 16 ? 192 : 128; }
+inline constexpr size_t kMmStagedLds = 40 * 1024;
 
-size_t match_mfma_lds_bytes(int step, int range, int group) {
+// LDS words of the MFMA matcher for `list` candidates per reference: the fp16
+// region (the exact keys over it), the exchange and lists, counters, and with
+// `staged` the FP32 region.
+static size_t mm_lds_words(int step, int range, size_t list, bool staged) {
     // the union of a 4 x 4 block's windows spans at most 3 step + 2 range + 1
     // candidate columns and rows
     const int span = 3 * step + 2 * range + 1;
     const int nt = (span + 15) >> 4;
+    const size_t reg = (std::max(static_cast<size_t>(span + 7) * static_cast<size_t>(h_mm_pitch.of[nt]), 16 * list) + 3) & ~static_cast<size_t>(3);
+    return reg + 8 * list + kMmCounters +
+           (staged ? static_cast<size_t>(span + 7) * mm_pitch32(nt) : 0);
+}
+
+// Regions staged in FP32 as well: those that leave four workgroups per CU.
+static bool mm_staged(int step, int range, size_t list) {
+    return mm_lds_words(step, range, list, true) * 4 <= kMmStagedLds;
+}
+
+size_t match_mfma_lds_bytes(int step, int range, int group) {
     const size_t list = static_cast<size_t>(mm_list(group));
-    const size_t reg = std::max(static_cast<size_t>(span + 7) * mm_pitch(nt), 16 * list);
-    return (reg + std::max(8 * list, static_cast<size_t>(2048)) + 66) * 4;
+    return mm_lds_words(step, range, list, mm_staged(step, range, list)) * 4;
 }
 
 bool match_mfma_fits(int block, int group, int step, int range, int width, int height) {
-    return block == 8 && group >= 1 && group <= 32 && width >= 8 && height >= 8 &&
+    return block == 8 && group >= 1 && group <= 32 && width >= 8 && height >= 8 && 3 * step + 2 * range + 1 <= 16 * kMmTiles &&
            match_mfma_lds_bytes(step, range, group) <= 160 * 1024;
 }
 
@@ -4467,20 +4714,25 @@ template <int B>
 static hipError_t launch_match_b(const MatchTable& t, int total_wg, size_t lds, int kind, hipStream_t s) {
     if (kind == 3) {
         if constexpr (B == 8) {
-            // One list length for the whole launch (the largest group's), so
-            // the LDS is sized here for every job at that length.
+            // One list length for the whole launch (the largest group's) and
+            // one staging form, so the LDS is sized here for every job.
             int gmax = 0;
             for (int j = 0; j < t.n; ++j) gmax = std::max(gmax, t.job[j].group);
+            const size_t list = static_cast<size_t>(mm_list(gmax));
+            bool staged = true;
+            for (int j = 0; j < t.n; ++j) staged &= mm_staged(t.job[j].grid.step, t.job[j].range, list);
+            lds = 0;
             for (int j = 0; j < t.n; ++j)
-                lds = std::max(lds, match_mfma_lds_bytes(t.job[j].grid.step, t.job[j].range, gmax));
+                lds = std::max(lds, mm_lds_words(t.job[j].grid.step, t.job[j].range, list, staged) * 4);
             if (lds > 160 * 1024) return hipErrorInvalidValue;
-            if (mm_list(gmax) == 256) {
-                allow_lds(&match_mfma_kernel<256>, lds);
-                match_mfma_kernel<256><<<total_wg, 256, lds, s>>>(t);
-            } else {
-                allow_lds(&match_mfma_kernel<128>, lds);
-                match_mfma_kernel<128><<<total_wg, 256, lds, s>>>(t);
-            }
+            auto launch = [&](auto kernel) {
+                allow_lds(kernel, lds);
+                kernel<<<total_wg, 256, lds, s>>>(t);
+            };
+            if (list == 192)
+                staged ? launch(&match_mfma_kernel<192, true>) : launch(&match_mfma_kernel<192, false>);
+            else
+                staged ? launch(&match_mfma_kernel<128, true>) : launch(&match_mfma_kernel<128, false>);
         } else {
             return hipErrorInvalidValue;
         }

@@ -62,7 +62,7 @@ int choose_match_kind(int block, int step, int range, int group, int width, int 
     const bool run_block = block == 1 || block == 2 || block == 4 || block == 8 || block == 12;
     const bool run = run_block && match_run_lds_bytes(block, step, range) <= kRunLdsBudget;
     if (match_path() != 1 && match_mfma_fits(block, group, step, range, width, height) &&
-        (match_path() == 2 || !run || (match_mfma_pays(step, range, group) && nref >= kMfmaMinRefs))) {
+        (match_path() == 2 || !run || match_mfma_pays(step, range, group, nref))) {
         *lds = match_mfma_lds_bytes(step, range, group);
         return 3;
     }
@@ -102,15 +102,27 @@ std::atomic<int> g_match_path{0};
 
 // The MFMA matcher scores every candidate of a 4 x 4 block's union window
 // (side 3 step + 2 range + 1) for all 16 references; the run matcher scores
-// each reference's own window. Measured on 1080p planes (block 8, group 8
-// and 16), the MFMA matcher is faster once the window side exceeds about
-// 3.3 steps (range >= 13 at step 8, >= 10 at step 4 or 3) and the frame has
-// enough references to fill the device (a 256 x 256 frame at step 3 does
-// not). The rule holds at group 32 as well (1080p YUV420, step 3, range 19,
-// groups 16 / 32: 7.1 ms per frame with both stages on the MFMA matcher
-// against 8.7 with the run matcher on the group-32 stage).
-bool match_mfma_pays(int step, int range, int group) {
-    return group <= 32 && range >= 10 && 3 * (2 * range + 1) > 10 * step;
+// each reference's own window, with its keys in registers up to range 17.
+// Measured at groups 8 / 16 / 32 (times of the run matcher over the MFMA's,
+// noisy frames; denoised ones within 0.1):
+//   range 18 and more: at step 3 1.5 / 1.3 / 1.5 on 128 x 96, 2.2 / 1.4 / 1.1
+//     on 256 x 256, 13 / 15 / 15 on 640 x 480 at range 24; at step 8, range 20
+//     1.5 / 1.8 / 2.1 on 128 x 96: any frame;
+//   ranges 10 to 17 on 1080p: at step 8 1.4 / 1.25 / 1.3 (range 10), 1.1 / 1.0
+//     / 1.1 (13), 1.5 / 1.5 / 1.8 (16), at step 3, range 16 2.7 / 2.6 / 3.2,
+//     and fewer references fill the chip less: at 961 (step 8) 0.7, at 6889
+//     (256 x 256, step 3) 1.2 / 1.2 / 1.05 (range 12), 1.7 / 1.7 / 1.4 (16);
+//   smaller ranges on 1080p: at step 4, range 9 1.4 / 1.2 / 1.05, at step 3
+//     1.55 / 1.25 / 1.1, at step 5 1.1 / 0.97 / 0.9, at step 8 1.0 / 0.8 / 0.8;
+//     18644 references at step 4 1.2 / 1.03 / 0.9.
+// Constant areas (the exact fallback takes them) cost the MFMA matcher more
+// than the run matcher at the smaller ranges: half a frame of them leaves
+// 0.9 of the run matcher's speed at step 3, range 9 and 1.1 to 2.2 above.
+bool match_mfma_pays(int step, int range, int group, long long nref) {
+    if (group > 32) return false;
+    if (range < 10) return step <= 4 && group <= 16 && nref >= 16384;
+    if (3 * (2 * range + 1) <= 7 * step) return false;  // the union is mostly gaps between the windows
+    return range >= 18 || nref >= (step <= 3 && group <= 16 ? 6144 : 16384);
 }
 
 int match_path() { return g_match_path.load(std::memory_order_relaxed); }
@@ -173,7 +185,7 @@ int plan_stage(nss_hip_bm3d* h, Stage& st) {
             if (st.plane[i].sigma != 0.f && st.plane[i].block == b) bk.planes[bk.nplanes++] = i;
         if (!bk.nplanes) continue;
         size_t run_lds = 0, wave_lds = 0, mfma_lds = 0;
-        bool mfma = match_path() != 1, mfma_pays = true;
+        bool mfma = match_path() != 1;
         long long nref = 0;
         for (int k = 0; k < bk.nplanes; ++k) {
             const StagePlane& sp = st.plane[bk.planes[k]];
@@ -182,12 +194,16 @@ int plan_stage(nss_hip_bm3d* h, Stage& st) {
             wave_lds = std::max(wave_lds, match_wave_lds_bytes(b, sp.range, true));
             mfma_lds = std::max(mfma_lds, match_mfma_lds_bytes(sp.step, sp.range, sp.group));
             mfma &= match_mfma_fits(b, sp.group, sp.step, sp.range, h->pw[i], h->ph[i]);
-            mfma_pays &= match_mfma_pays(sp.step, sp.range, sp.group);
             const Grid gr = make_grid(h->pw[i], h->ph[i], b, sp.step);
             nref += static_cast<long long>(gr.nx) * gr.ny;
         }
         const bool run = b <= 12 && run_lds <= kRunLdsBudget;
-        if (mfma && (match_path() == 2 || !run || (mfma_pays && nref >= kMfmaMinRefs))) {
+        bool mfma_pays = true;
+        for (int k = 0; k < bk.nplanes; ++k) {
+            const StagePlane& sp = st.plane[bk.planes[k]];
+            mfma_pays &= match_mfma_pays(sp.step, sp.range, sp.group, nref);
+        }
+        if (mfma && (match_path() == 2 || !run || mfma_pays)) {
             bk.match_kind = 3;
             bk.match_lds = mfma_lds;
         } else if (run) {
