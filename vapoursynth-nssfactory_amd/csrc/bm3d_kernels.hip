@@ -1793,6 +1793,67 @@ __device__ inline unsigned long long to_fixed(float v) {
     return static_cast<unsigned long long>(__float2ll_rn(v * 4294967296.0f));
 }
 
+// to_fixed of N values. Below 2^19 the conversion is one double addition: at
+// 1.5 * 2^20 a double's unit is 2^-32, so the sum rounds to nearest even there
+// as __float2ll_rn does, and the words less the constant's are the integer.
+// Three operations instead of twelve (the cast's high and low words), which
+// were a sixth of the group filters' VALU time: 1080p YUV420 at group 8 hard
+// 45.3 -> 42.6 us, Wiener (with quotient()) 63.0 -> 57.3 us; group 32 Wiener
+// at step 3 1609 -> 1489 us. Larger or non-finite
+// values (one test of the magnitudes' sum) take the cast.
+template <int N>
+__device__ __forceinline__ void to_fixed_n(const float (&v)[N], unsigned long long (&o)[N]) {
+    float mag = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) mag += fabsf(v[i]);
+    if (mag < 524288.f) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            o[i] = static_cast<unsigned long long>(__double_as_longlong(static_cast<double>(v[i]) + 1572864.0)) -
+                   0x4138000000000000ull;
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) o[i] = to_fixed(v[i]);
+    }
+}
+
+// n / d, correctly rounded, for d in [2^-60, 2^62] and 0 <= n <= d: Newton's
+// step on the reciprocal and two residual corrections (the operations of the
+// full division without its scaling and special cases).
+__device__ __forceinline__ float quotient(float n, float d) {
+    float y = __builtin_amdgcn_rcpf(d);
+    y = fmaf(fmaf(-d, y, 1.f), y, y);
+    float q = n * y;
+    q = fmaf(fmaf(-d, q, n), y, q);
+    return fmaf(fmaf(-d, q, n), y, q);
+}
+
+// Wiener gains r^2 / (r^2 + sig2) applied to a lane's G coefficients (lane 0's
+// first, the group's mean, keeps 1); the sum of their squares is returned.
+template <int G>
+__device__ __forceinline__ float wiener_shrink(float (&c)[G], const float (&r)[G], float sig2, int lane) {
+    float mag = 0.f, w2 = 0.f;
+#pragma unroll
+    for (int j = 0; j < G; ++j) mag += fabsf(r[j]);
+    auto shrink = [&](auto gain) {
+#pragma unroll
+        for (int j = 0; j < G; ++j) {
+            float w = 1.f;
+            if (!(lane == 0 && j == 0)) {
+                const float r2 = r[j] * r[j];
+                w = gain(r2, r2 + sig2);
+            }
+            c[j] *= w;
+            w2 = fmaf(w, w, w2);
+        }
+    };
+    if (mag < 1073741824.f && sig2 > 0x1p-60f)
+        shrink([](float n, float d) { return quotient(n, d); });
+    else
+        shrink([](float n, float d) { return d > 0.f ? n / d : 0.f; });
+    return w2;
+}
+
 __device__ inline void lds_add(unsigned long long* p, unsigned long long v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -2143,20 +2204,11 @@ __global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
         }
         int kept = 0;
         float w2 = 0.f;
+        if constexpr (WIENER) w2 = wiener_shrink<G>(c, r, sig2, lane);
 #pragma unroll
         for (int j = 0; j < G; ++j) {
-            const bool dc = (lane == 0 && j == 0);
-            if constexpr (WIENER) {
-                float w = 1.f;
-                if (!dc) {
-                    const float r2 = r[j] * r[j];
-                    const float den = r2 + sig2;
-                    w = den > 0.f ? r2 / den : 0.f;
-                }
-                c[j] *= w;
-                w2 = fmaf(w, w, w2);
-            } else {
-                if (!dc && fabsf(c[j]) < thr)
+            if constexpr (!WIENER) {
+                if (!(lane == 0 && j == 0) && fabsf(c[j]) < thr)
                     c[j] = 0.f;
                 else
                     ++kept;
@@ -2183,8 +2235,13 @@ __global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
             if (p < k) {
                 const int lx = rec[p].x - ax0, ly = rec[p].y - ay0;
                 unsigned long long* row = num + (ly + y) * aw + lx;
+                float wu[8];
 #pragma unroll
-                for (int x = 0; x < 8; ++x) lds_add(row + x, to_fixed(w * u[m][x]));
+                for (int x = 0; x < 8; ++x) wu[x] = w * u[m][x];
+                unsigned long long fx[8];
+                to_fixed_n<8>(wu, fx);
+#pragma unroll
+                for (int x = 0; x < 8; ++x) lds_add(row + x, fx[x]);
             }
         }
         if (lane == 0) {
@@ -2729,8 +2786,13 @@ __global__ __launch_bounds__(256) void filter_tile_mfma_kernel(FilterTable tab) 
                 const float wq = w / s[gsel];
                 const float wm = w * mu[gsel];  // the centre, added back
                 unsigned long long* cell = num + (ly + y0) * aw + lx + px;
+                float wx[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) lds_add(cell + j * aw, to_fixed(fmaf(wq, xo[q][j], wm)));
+                for (int j = 0; j < 4; ++j) wx[j] = fmaf(wq, xo[q][j], wm);
+                unsigned long long fx[4];
+                to_fixed_n<4>(wx, fx);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) lds_add(cell + j * aw, fx[j]);
             }
         }
         // the unit's group weights (two groups of 8 or one of 16)
@@ -3137,20 +3199,11 @@ __global__ __launch_bounds__(256) void filter_temporal_b8_kernel(TFilterTable ta
     const float sig2 = jb.sigma * jb.sigma;
     int kept = 0;
     float w2 = 0.f;
+    if constexpr (WIENER) w2 = wiener_shrink<G>(c, r, sig2, lane);
 #pragma unroll
     for (int j = 0; j < G; ++j) {
-        const bool dc = (lane == 0 && j == 0);
-        if constexpr (WIENER) {
-            float w = 1.f;
-            if (!dc) {
-                const float r2 = r[j] * r[j];
-                const float den = r2 + sig2;
-                w = den > 0.f ? r2 / den : 0.f;
-            }
-            c[j] *= w;
-            w2 = fmaf(w, w, w2);
-        } else {
-            if (!dc && fabsf(c[j]) < thr)
+        if constexpr (!WIENER) {
+            if (!(lane == 0 && j == 0) && fabsf(c[j]) < thr)
                 c[j] = 0.f;
             else
                 ++kept;
@@ -3347,20 +3400,11 @@ __global__ __launch_bounds__(512) void filter_temporal_tile_kernel(TTileTable ta
             if (g + kTTileWaves < cur.ngroups) gather(cur, g + kTTileWaves, v, vr);
             int kept = 0;
             float w2 = 0.f;
+            if constexpr (WIENER) w2 = wiener_shrink<G>(c, r, sig2, lane);
 #pragma unroll
             for (int j = 0; j < G; ++j) {
-                const bool dc = (lane == 0 && j == 0);
-                if constexpr (WIENER) {
-                    float w = 1.f;
-                    if (!dc) {
-                        const float r2 = r[j] * r[j];
-                        const float den = r2 + sig2;
-                        w = den > 0.f ? r2 / den : 0.f;
-                    }
-                    c[j] *= w;
-                    w2 = fmaf(w, w, w2);
-                } else {
-                    if (!dc && fabsf(c[j]) < thr)
+                if constexpr (!WIENER) {
+                    if (!(lane == 0 && j == 0) && fabsf(c[j]) < thr)
                         c[j] = 0.f;
                     else
                         ++kept;
@@ -3392,8 +3436,13 @@ __global__ __launch_bounds__(512) void filter_temporal_tile_kernel(TTileTable ta
                     // than written out of bounds.
                     if (lx >= 0 && ly >= 0 && lx <= q.aw - B && ly <= q.ah - B) {
                         unsigned long long* row = acc + q.off + (ly + y) * q.aw + lx;
+                        float wu[8];
 #pragma unroll
-                        for (int x = 0; x < 8; ++x) lds_add(row + x, to_fixed(w * u[m][x]));
+                        for (int x = 0; x < 8; ++x) wu[x] = w * u[m][x];
+                        unsigned long long fx[8];
+                        to_fixed_n<8>(wu, fx);
+#pragma unroll
+                        for (int x = 0; x < 8; ++x) lds_add(row + x, fx[x]);
                         if (y == 0) {
                             if (jb.corners)
                                 atomicAdd(jb.corners +
@@ -4581,12 +4630,16 @@ __global__ __launch_bounds__(256, 4) void gram_group_tile_kernel(WnnmTable tab) 
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
                     x[4 * s / N] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[u][s], b[t][s], x[4 * s / N], 0, 0, 0);
+                float wx[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) wx[j] = lane_f32(wt, N * (u * HN + 4 * j / N)) * (x[4 * j / N][j] + mu[4 * j / N]);
+                unsigned long long fx[4];
+                to_fixed_n<4>(wx, fx);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int h = 4 * j / N;
-                    const float w = lane_f32(wt, N * (u * HN + h));
                     unsigned long long* cell = acc + (rec[u][j].y - ay0 + 2 * t + (n >> 3)) * aw + rec[u][j].x - ax0 + (n & 7);
-                    if (g0 + u * HN + h < ngroups) lds_add(cell, to_fixed(w * (x[h][j] + mu[h])));
+                    if (g0 + u * HN + h < ngroups) lds_add(cell, fx[j]);
                 }
             }
         }

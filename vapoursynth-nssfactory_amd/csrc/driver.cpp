@@ -111,7 +111,7 @@ std::atomic<int> g_match_path{0};
 //   ranges 10 to 17 on 1080p: at step 8 1.4 / 1.25 / 1.3 (range 10), 1.1 / 1.0
 //     / 1.1 (13), 1.5 / 1.5 / 1.8 (16), at step 3, range 16 2.7 / 2.6 / 3.2,
 //     and fewer references fill the chip less: at 961 (step 8) 0.7, at 6889
-//     (256 x 256, step 3) 1.2 / 1.2 / 1.05 (range 12), 1.7 / 1.7 / 1.4 (16);
+//     (256 x 256, step 3) between 0.95 and 1.7 with the content;
 //   smaller ranges on 1080p: at step 4, range 9 1.4 / 1.2 / 1.05, at step 3
 //     1.55 / 1.25 / 1.1, at step 5 1.1 / 0.97 / 0.9, at step 8 1.0 / 0.8 / 0.8;
 //     18644 references at step 4 1.2 / 1.03 / 0.9.
@@ -122,7 +122,7 @@ bool match_mfma_pays(int step, int range, int group, long long nref) {
     if (group > 32) return false;
     if (range < 10) return step <= 4 && group <= 16 && nref >= 16384;
     if (3 * (2 * range + 1) <= 7 * step) return false;  // the union is mostly gaps between the windows
-    return range >= 18 || nref >= (step <= 3 && group <= 16 ? 6144 : 16384);
+    return range >= 18 || nref >= 16384;
 }
 
 int match_path() { return g_match_path.load(std::memory_order_relaxed); }
