@@ -2146,7 +2146,7 @@ __device__ inline void gather_rows_b8(const float* plane, int stride, const Matc
 // Tile kernel for block 8: LDS = num [ah][aw] int64 | match records of the
 // tile | per-wave transpose buffers.
 template <int G, bool WIENER>
-__global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
+__global__ __launch_bounds__(G <= 16 ? 1024 : 256) void filter_tile_b8_kernel(FilterTable tab) {
     extern __shared__ __align__(16) unsigned long long acc[];
     constexpr int B = 8;
     constexpr int M = G / 8;
@@ -2166,16 +2166,17 @@ __global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
     int* cnt = reinterpret_cast<int*>(recs + tg.tw * tg.th * G);
     float* scratch = reinterpret_cast<float*>(cnt + ((tg.tw * tg.th + 3) & ~3));
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int nt = static_cast<int>(blockDim.x), waves = nt >> 6;
     float* T = scratch + wave * (G * kTs);
-    for (int e = threadIdx.x; e < aw * ah; e += 256) acc[e] = 0ull;
+    for (int e = threadIdx.x; e < aw * ah; e += nt) acc[e] = 0ull;
     // The tile's match records and counts, row by row of the grid.
-    for (int e = threadIdx.x; e < ngroups * G; e += 256) {
+    for (int e = threadIdx.x; e < ngroups * G; e += nt) {
         const int g = e / G, j = e - g * G;
         const int gj = g / ni, gi = g - gj * ni;
         const int rid = (j_begin + gj - jb.grid.row0) * jb.grid.nx + i_begin + gi;
         recs[e] = jb.matches[static_cast<size_t>(rid) * G + j];
     }
-    for (int g = threadIdx.x; g < ngroups; g += 256) {
+    for (int g = threadIdx.x; g < ngroups; g += nt) {
         const int gj = g / ni, gi = g - gj * ni;
         cnt[g] = jb.counts[(j_begin + gj - jb.grid.row0) * jb.grid.nx + i_begin + gi];
     }
@@ -2189,7 +2190,7 @@ __global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
         gather_rows_b8<G>(jb.src, jb.stride, recs + g * G, cnt[g], lane, v);
         if constexpr (WIENER) gather_rows_b8<G>(jb.wref, jb.wref_stride, recs + g * G, cnt[g], lane, vr);
     }
-    for (; g < ngroups; g += 4) {
+    for (; g < ngroups; g += waves) {
         const int k = cnt[g];
         const MatchRec* rec = recs + g * G;
         float c[G];
@@ -2197,7 +2198,7 @@ __global__ __launch_bounds__(256) void filter_tile_b8_kernel(FilterTable tab) {
         forward_b8<G>(v, c, T, lane);
         if constexpr (WIENER) forward_b8<G>(vr, r, T, lane);
         // Prefetch the next group's patches while this one is filtered.
-        const int gn = g + 4;
+        const int gn = g + waves;
         if (gn < ngroups) {
             gather_rows_b8<G>(jb.src, jb.stride, recs + gn * G, cnt[gn], lane, v);
             if constexpr (WIENER) gather_rows_b8<G>(jb.wref, jb.wref_stride, recs + gn * G, cnt[gn], lane, vr);
@@ -3590,25 +3591,27 @@ __global__ __launch_bounds__(256) void finish_temporal_tiles_kernel(TFinishTable
 // conversion and num / den in double rounded to float (the atomic path's
 // formula, finish_corner_kernel). Otherwise the temporal slot partials
 // (floats) in slice mode.
-template <bool EXACT>
-__global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
+template <bool EXACT, int PX>
+__global__ __launch_bounds__(1024 / PX) void finish_tiles_kernel(FinishTable tab) {
     extern __shared__ __align__(16) unsigned long long fsm[];
     // XCD-contiguous blocks: neighbouring blocks read the same tile partial
     // lines through one L2.
     const int lb = xcd_block();
+    constexpr int nt = 1024 / PX;
+    constexpr int U = PX == 1 ? 4 : 2;  // tiles' partials in flight
     const FinishJob& jb = tab.job[find_job(tab, lb)];
     const int t = lb - jb.wg_begin;
     const int bx0 = (t % jb.tiles_x) * 64, by0 = jb.py0 + (t / jb.tiles_x) * 16;
-    const int x0 = bx0 + (threadIdx.x & 15) * 4;
-    const int y = by0 + (threadIdx.x >> 4);
+    const int x0 = bx0 + (threadIdx.x & (64 / PX - 1)) * PX;
+    const int y = by0 + threadIdx.x / (64 / PX);
     const int B = jb.block, s = jb.step, r = jb.range;
-    long long dw[4] = {0, 0, 0, 0};  // EXACT: the weights' sums
+    long long dw[PX] = {};  // EXACT: the weights' sums
     if constexpr (EXACT) {
         const int CW = 64 + B - 1, CH = 16 + B - 1;
         const int cx0 = bx0 - B + 1, cy0 = by0 - B + 1;  // corner tile origin
         unsigned long long* ct = fsm;                     // [CH][CW] corner weights
         unsigned long long* hs = fsm + CH * CW;           // [CH][64] horizontal B-wide sums
-        for (int e = threadIdx.x; e < CH * CW; e += 256) ct[e] = 0ull;
+        for (int e = threadIdx.x; e < CH * CW; e += nt) ct[e] = 0ull;
         __syncthreads();
         // The references whose windows (reference +- range, clamped) reach
         // the corner tile, of the grid rows the records hold.
@@ -3624,19 +3627,19 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
         // four (reference, record) pairs per thread and step, every load of
         // them issued before any is used (a reference holds G records; the
         // ones at or beyond its count are read and not used)
-        for (int e0 = threadIdx.x; e0 < pairs; e0 += 1024) {
+        for (int e0 = threadIdx.x; e0 < pairs; e0 += 4 * nt) {
             int cnt[4], kk[4], ox[4], oy[4];
             unsigned long long wgt[4];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int e = min(e0 + 256 * u, pairs - 1);
+                const int e = min(e0 + nt * u, pairs - 1);
                 const int ref = e / G, k = e - ref * G;
                 const int rj = ref / ni, ri = ref - rj * ni;
                 const int rid = (a_lo - g.row0 + rj) * g.nx + i_lo + ri;
                 cnt[u] = jb.counts[rid];
                 const MatchRec m = jb.matches[static_cast<size_t>(rid) * G + k];
                 wgt[u] = jb.gweight[rid];
-                kk[u] = e0 + 256 * u < pairs ? k : G;
+                kk[u] = e0 + nt * u < pairs ? k : G;
                 ox[u] = m.x - cx0;
                 oy[u] = m.y - cy0;
             }
@@ -3650,7 +3653,7 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
         // hs[row][x] = sum of ct[row][x .. x + B - 1], then the B-high sums
         // into the corner tile's area, den[yr][x]: a wave's lanes take 64
         // consecutive x of one row (bank-conflict-free reads and writes)
-        for (int e = threadIdx.x; e < CH * 64; e += 256) {
+        for (int e = threadIdx.x; e < CH * 64; e += nt) {
             const int row = e >> 6, x = e & 63;
             const unsigned long long* cr = ct + row * CW + x;
             unsigned long long sum = 0;
@@ -3659,7 +3662,7 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
         }
         __syncthreads();
         unsigned long long* den = ct;  // [16][64]
-        for (int e = threadIdx.x; e < 16 * 64; e += 256) {
+        for (int e = threadIdx.x; e < 16 * 64; e += nt) {
             const unsigned long long* hc = hs + e;
             unsigned long long sum = 0;
             for (int a = 0; a < B; ++a) sum += hc[a * 64];
@@ -3669,11 +3672,11 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
         // the weight at (x, y): corners (x - B + 1 .. x, y - B + 1 .. y)
         const unsigned long long* dr = den + (y - by0) * 64 + (x0 - bx0);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) dw[q] = static_cast<long long>(dr[q]);
+        for (int q = 0; q < PX; ++q) dw[q] = static_cast<long long>(dr[q]);
     }
     if (x0 >= jb.width || y >= jb.height) return;
     const TileGeom& tg = jb.tiles;
-    const int xr = min(x0 + 3, jb.width - 1);
+    const int xr = min(x0 + PX - 1, jb.width - 1);
     int txh = min(tg.ntx - 1, (xr + r) / (tg.tw * s));
     while (txh + 1 < tg.ntx && tg.ax0(txh + 1, jb.width, B, s, r) <= xr) ++txh;
     int tyh = min(tg.nty - 1, (y + r) / (tg.th * s));
@@ -3683,36 +3686,38 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
     const int ty_lo = batch ? jb.ty0 : 0;
     if (batch) tyh = min(tyh, jb.ty1 - 1);
     using Acc = typename std::conditional<EXACT, long long, float>::type;
-    Acc n[4] = {0, 0, 0, 0}, d[4] = {0, 0, 0, 0};
+    Acc n[PX] = {}, d[PX] = {};
     const size_t area = static_cast<size_t>(tg.pitch) * tg.ah;
     // The covering tiles are the rectangle [tyl, tyh] x [txl, txh]; walked
-    // in descending (ty, tx) order, two tiles' partials are loaded before
-    // either is added, so their memory latencies overlap (four at a time
-    // need 106 VGPRs and ran slower).
+    // in descending (ty, tx) order, U tiles' partials are loaded before any is
+    // added, so their memory latencies overlap (four at a time with four pixels
+    // each need 106 VGPRs and ran slower).
     int tyl = tyh + 1;
     while (tyl - 1 >= ty_lo && y - tg.ay0(tyl - 1, jb.height, B, s, r) < tg.ah) --tyl;
     int txl = txh + 1;
     while (txl - 1 >= 0 && tg.ax0(txl - 1, jb.width, B, s, r) + tg.aw > x0) --txl;
     const int nx = txh - txl + 1;
     const int count = tyl <= tyh ? (tyh - tyl + 1) * nx : 0;
-    for (int k0 = 0; k0 < count; k0 += 2) {
-        Acc pn[2][4], pd[2][4];
-        int lo[2];
+    for (int k0 = 0; k0 < count; k0 += U) {
+        Acc pn[U][PX], pd[U][PX];
+        int lo[U];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < U; ++u) {
             const int k = k0 + u;
-            lo[u] = x0 + 4;  // no pixel of the four inside
+            lo[u] = x0 + PX;  // no pixel inside
 #pragma unroll
-            for (int i = 0; i < 4; ++i) pn[u][i] = pd[u][i] = Acc(0);
+            for (int i = 0; i < PX; ++i) pn[u][i] = pd[u][i] = Acc(0);
             if (k < count) {
                 const int ty = tyh - k / nx, tx = txh - k % nx;
                 const int oy = y - tg.ay0(ty, jb.height, B, s, r);
                 const int ax0 = tg.ax0(tx, jb.width, B, s, r);
                 lo[u] = ax0;
-                // column of x0: a multiple of 4 in [0, pitch - 4]
+                // column of x0: a multiple of PX in [0, pitch - PX]
                 const size_t o = (static_cast<size_t>(ty - ty_lo) * tg.ntx + tx) * area +
                                  static_cast<size_t>(oy) * tg.pitch + (x0 - ax0 + (ax0 & 3));
-                if constexpr (EXACT) {
+                if constexpr (EXACT && PX == 1) {
+                    pn[u][0] = static_cast<long long>(jb.exact_num[o]);
+                } else if constexpr (EXACT) {
                     const longlong2* qn =
                         static_cast<const longlong2*>(__builtin_assume_aligned(jb.exact_num + o, 32));
                     const longlong2 n0 = qn[0], n1 = qn[1];
@@ -3721,14 +3726,14 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
                     const f32x4 vn = *reinterpret_cast<const f32x4*>(jb.part_num + o);
                     const f32x4 vd = *reinterpret_cast<const f32x4*>(jb.part_den + o);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) pn[u][i] = vn[i], pd[u][i] = vd[i];
+                    for (int i = 0; i < PX; ++i) pn[u][i] = vn[i], pd[u][i] = vd[i];
                 }
             }
         }
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < PX; ++i) {
                 const bool in = k0 + u < count && static_cast<unsigned>(x0 + i - lo[u]) < static_cast<unsigned>(tg.aw);
                 n[i] += in ? pn[u][i] : Acc(0);
                 d[i] += in ? pd[u][i] : Acc(0);
@@ -3736,12 +3741,12 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
     }
     if constexpr (EXACT) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[i] = dw[i];
+        for (int i = 0; i < PX; ++i) d[i] = dw[i];
         if (batch) {
             long long* an = jb.acc_num + static_cast<size_t>(y) * jb.width;
             long long* ad = jb.acc_den + static_cast<size_t>(y) * jb.width;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < PX; ++i)
                 if (x0 + i < jb.width) {
                     an[x0 + i] += n[i];
                     ad[x0 + i] += d[i];
@@ -3753,7 +3758,7 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
     if (jb.dst_den) {
         float* dd = jb.dst_den + static_cast<size_t>(y) * jb.dstride;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < PX; ++i)
             if (x0 + i < jb.width) {
                 if constexpr (EXACT) {
                     dst[x0 + i] = static_cast<float>(static_cast<double>(n[i]) * (1.0 / 4294967296.0));
@@ -3767,7 +3772,7 @@ __global__ __launch_bounds__(256) void finish_tiles_kernel(FinishTable tab) {
     }
     const float* src = jb.src + static_cast<size_t>(y) * jb.sstride;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < PX; ++i)
         if (x0 + i < jb.width) {
             if constexpr (EXACT)
                 dst[x0 + i] = d[i] > 0 ? static_cast<float>(static_cast<double>(n[i]) / static_cast<double>(d[i]))
@@ -4892,15 +4897,38 @@ static hipError_t launch_filter_b(const FilterTable& t, int total_wg, size_t lds
     return hipGetLastError();
 }
 
+// A launch of up to 256 workgroups has a CU for each: 16 waves share a filter
+// tile's groups, and the finish takes one pixel per thread. 128 x 96 YUV420,
+// group 8: hard 10.8 -> 7.1 us, Wiener 12.5 -> 8.4; finish of 256 x 256 at step
+// 3, group 16: 22.7 -> 19.6. Above that, eight waves per tile serve the hard
+// stage (1080p YUV420 43.5 -> 42.0 us, 256 x 256 at step 3, group 16 18.6 ->
+// 16.8) and four the Wiener stage (57.3 us against 60.8: its registers leave
+// the fifth to eighth wave of a SIMD out).
+inline constexpr int kFinishAloneBlocks = 256;
+inline constexpr int kFilterAloneTiles = 256;
+inline constexpr int kFilterWaves = 8;
+
 template <int G>
 static hipError_t launch_filter_b8(const FilterTable& t, int total_wg, size_t lds, bool wiener, hipStream_t s) {
-    if (wiener) {
-        allow_lds(&filter_tile_b8_kernel<G, true>, lds);
-        filter_tile_b8_kernel<G, true><<<total_wg, 256, lds, s>>>(t);
-    } else {
-        allow_lds(&filter_tile_b8_kernel<G, false>, lds);
-        filter_tile_b8_kernel<G, false><<<total_wg, 256, lds, s>>>(t);
+    int waves = 4;  // what lds holds transpose buffers for
+    if (G <= 16) {
+        const size_t each = static_cast<size_t>(G) * kTs * 4;
+        int groups = 1;
+        for (int j = 0; j < t.n; ++j) groups = std::max(groups, t.job[j].tiles.tw * t.job[j].tiles.th);
+        const int want = total_wg <= kFilterAloneTiles ? 16 : wiener ? 4 : kFilterWaves;
+        while (2 * waves <= want && waves < groups && lds + waves * each <= (want == 16 ? 160 : 80) * 1024) {
+            lds += waves * each;
+            waves *= 2;
+        }
     }
+    const auto launch = [&](auto kernel) {
+        allow_lds(kernel, lds);
+        kernel<<<total_wg, 64 * waves, lds, s>>>(t);
+    };
+    if (wiener)
+        launch(&filter_tile_b8_kernel<G, true>);
+    else
+        launch(&filter_tile_b8_kernel<G, false>);
     return hipGetLastError();
 }
 
@@ -4967,10 +4995,15 @@ hipError_t launch_finish(int block, const FinishTable& t, int total_wg, bool til
             int bmax = 1;
             for (int k = 0; k < t.n; ++k) bmax = std::max(bmax, t.job[k].block);
             const size_t lds = finish_tiles_lds_bytes(bmax);
-            allow_lds(&finish_tiles_kernel<true>, lds);
-            finish_tiles_kernel<true><<<total_wg, 256, lds, s>>>(t);
+            if (total_wg <= kFinishAloneBlocks) {
+                allow_lds(&finish_tiles_kernel<true, 1>, lds);
+                finish_tiles_kernel<true, 1><<<total_wg, 1024, lds, s>>>(t);
+            } else {
+                allow_lds(&finish_tiles_kernel<true, 4>, lds);
+                finish_tiles_kernel<true, 4><<<total_wg, 256, lds, s>>>(t);
+            }
         } else {
-            finish_tiles_kernel<false><<<total_wg, 256, 0, s>>>(t);
+            finish_tiles_kernel<false, 4><<<total_wg, 256, 0, s>>>(t);
         }
         return hipGetLastError();
     }
