@@ -1886,8 +1886,9 @@ __device__ inline void partials_out_float(int aw, int ah, int pitch, const unsig
     const int cw = aw - B + 1, ch = ah - B + 1;
     const int nt = static_cast<int>(blockDim.x);
     if (!pd) {  // numerator only (the weights went to the frame's corner plane)
+        const float inv = 1.f / static_cast<float>(aw);
         for (int e = threadIdx.x; e < aw * ah; e += nt) {
-            const int y = e / aw, x = e - (e / aw) * aw;
+            const int y = div_small(e, inv), x = e - y * aw;
             pn[y * pitch + x] =
                 static_cast<float>(static_cast<double>(static_cast<long long>(num[e])) * (1.0 / 4294967296.0));
         }
@@ -3308,7 +3309,7 @@ __device__ inline void ttile_gather(const TTileJob& jb, const MatchRec* rec, int
 }
 
 template <int G, bool WIENER>
-__global__ __launch_bounds__(512) void filter_temporal_tile_kernel(TTileTable tab, int total_tiles) {
+__global__ __launch_bounds__(G == 8 ? 1024 : 512) void filter_temporal_tile_kernel(TTileTable tab, int total_tiles) {
     extern __shared__ __align__(16) unsigned long long smem64[];
     constexpr int B = 8;
     constexpr int M = G / 8;
@@ -3317,13 +3318,14 @@ __global__ __launch_bounds__(512) void filter_temporal_tile_kernel(TTileTable ta
     const int hi = static_cast<int>(static_cast<long long>(L + 1) * total_tiles / nb);
     if (lo >= hi) return;
     // Groups per tile (one tile shape per launch; tw * th * G <= 512, one
-    // record per thread).
+    // record per thread at most).
     const int cap = tab.job[0].tiles[0].tw * tab.job[0].tiles[0].th;
     MatchRec* recs = reinterpret_cast<MatchRec*>(smem64);
     int* cnt = reinterpret_cast<int*>(recs + cap * G);
     unsigned long long* acc = reinterpret_cast<unsigned long long*>(cnt + ((cap + 3) & ~3));
     __shared__ SlotLds sl[kMaxTileSlots];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int nt = static_cast<int>(blockDim.x), waves = nt >> 6;
     const int gb = lane >> 3, y = lane & 7;
 
     // Thread e's record (e < ngroups G) and count (e < ngroups) of tile a,
@@ -3387,18 +3389,18 @@ __global__ __launch_bounds__(512) void filter_temporal_tile_kernel(TTileTable ta
         }
         float* scratch = reinterpret_cast<float*>(acc + ((total + 1) & ~1));
         float* T = scratch + wave * (G * kTs);
-        for (int e = threadIdx.x; e < total; e += 512) acc[e] = 0ull;
+        for (int e = threadIdx.x; e < total; e += nt) acc[e] = 0ull;
         __syncthreads();
 
         const float thr = 2.7f * jb.sigma;  // include/nss/params.hpp:46 kBmHardLambda
         const float sig2 = jb.sigma * jb.sigma;
-        for (int g = wave; g < cur.ngroups; g += kTTileWaves) {
+        for (int g = wave; g < cur.ngroups; g += waves) {
             const int k = cnt[g];
             const MatchRec* rec = recs + g * G;
             float c[G], r[G];
             forward_b8<G>(v, c, T, lane);
             if constexpr (WIENER) forward_b8<G>(vr, r, T, lane);
-            if (g + kTTileWaves < cur.ngroups) gather(cur, g + kTTileWaves, v, vr);
+            if (g + waves < cur.ngroups) gather(cur, g + waves, v, vr);
             int kept = 0;
             float w2 = 0.f;
             if constexpr (WIENER) w2 = wiener_shrink<G>(c, r, sig2, lane);
@@ -5107,24 +5109,34 @@ size_t filter_temporal_tile_lds_bytes(int group, const TileGeom* g, int ns, bool
 
 // Persistent grid: as many workgroups as the device holds at once (at most
 // one per tile).
-template <typename Kernel>
+template <int G, typename Kernel>
 static hipError_t launch_persistent_ttile(Kernel k, const TTileTable& t, int tiles, size_t lds, hipStream_t s) {
     allow_lds(k, lds);
-    int dev = 0, cus = 0, per_cu = 0;
+    int dev = 0, cus = 0, per_cu = 0, threads = 64 * kTTileWaves;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 512, lds);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, lds);
     if (e != hipSuccess) return e;
+    // Slots that leave room for one workgroup only: 16 waves share its tiles
+    // (two per SIMD were a third of the VALU's rate; 1080p YUV420, radius 1,
+    // group 8: hard 126 -> 102 us, Wiener 183 -> 169 us per launch; groups of
+    // 16 would spill at 128 registers).
+    const size_t more = static_cast<size_t>(kTTileWaves) * G * kTs * 4;
+    if (G == 8 && per_cu <= 1 && lds + more <= 160 * 1024) {
+        lds += more;
+        threads *= 2;
+        allow_lds(k, lds);
+    }
     const int grid = std::max(1, std::min(tiles, std::max(cus, 1) * std::max(per_cu, 1)));
-    k<<<grid, 512, lds, s>>>(t, tiles);
+    k<<<grid, threads, lds, s>>>(t, tiles);
     return hipGetLastError();
 }
 
 template <int G>
 static hipError_t launch_ttile(const TTileTable& t, int tiles, size_t lds, bool wiener, hipStream_t s) {
     if (t.job[0].tiles[0].tw * t.job[0].tiles[0].th * G > 512) return hipErrorInvalidValue;
-    return wiener ? launch_persistent_ttile(&filter_temporal_tile_kernel<G, true>, t, tiles, lds, s)
-                  : launch_persistent_ttile(&filter_temporal_tile_kernel<G, false>, t, tiles, lds, s);
+    return wiener ? launch_persistent_ttile<G>(&filter_temporal_tile_kernel<G, true>, t, tiles, lds, s)
+                  : launch_persistent_ttile<G>(&filter_temporal_tile_kernel<G, false>, t, tiles, lds, s);
 }
 
 hipError_t launch_filter_temporal_tiles(int group, const TTileTable& t, int total_wg, size_t lds, bool wiener,
