@@ -2947,6 +2947,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void pr
             };
             const int R = W + B - 1, P = pred_region_pitch(W, B), SW = (W + 2) / 3;
             const bool staged = cells <= tab.chunk && nc * R * P <= tab.region;
+            // A layer of up to 64 strips keeps its keys in registers, three a
+            // lane: the winners come from wave minima instead of passes over
+            // the keys in LDS (1080p YUV420, two windows of 9 x 9: 142 -> 126
+            // us per launch, with the strips' divisions by reciprocals).
+            bool held = false;
+            unsigned long long strip[3] = {~0ull, ~0ull, ~0ull};
             if (staged) {
                 // Window w's pixels (rows y_w - ps .., columns x_w - ps ..) at
                 // region[w R P + j P + i]. Columns from R on and pixels off the
@@ -2956,7 +2962,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void pr
                 // Lanes cover 64 / P rows of P columns per step (P <= 64), or
                 // one row in steps of 64 columns.
                 const int rows_per = P <= 64 ? 64 / P : 1;
-                const int lr = P <= 64 ? lane / P : 0, li = P <= 64 ? lane - lr * P : lane;
+                const int lr = P <= 64 ? div_small(lane, __builtin_amdgcn_rcpf(static_cast<float>(P))) : 0;
+                const int li = P <= 64 ? lane - lr * P : lane;
                 for (int w = 0; w < nc; ++w) {
                     const int cw = centers[w];
                     const int y0 = (cw >> 13) - ps, x0 = (cw & 8191) - ps;
@@ -2992,9 +2999,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void pr
                 }
                 __syncthreads();
                 const int strips = nc * W * SW;
+                held = strips <= 64;
+                const float inv_ws = __builtin_amdgcn_rcpf(static_cast<float>(W * SW));
+                const float inv_s = __builtin_amdgcn_rcpf(static_cast<float>(SW));
                 for (int sidx = lane; sidx < strips; sidx += 64) {
-                    const int w = sidx / (W * SW), o = sidx - w * (W * SW);
-                    const int dy = o / SW, dx0 = 3 * (o - dy * SW);
+                    // (below 2^20 strips: exact from the hardware reciprocals)
+                    const int w = div_small(sidx, inv_ws), o = sidx - w * (W * SW);
+                    const int dy = div_small(o, inv_s), dx0 = 3 * (o - dy * SW);
                     const float* rb = region + w * (R * P) + dy * P + dx0;
                     float a0 = 0.f, a1 = 0.f, a2 = 0.f;
 #pragma unroll 1
@@ -3019,16 +3030,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void pr
                         if (dx < W) {
                             const int x = (cw & 8191) - ps + dx;
                             const float a = q == 0 ? a0 : q == 1 ? a1 : a2;
-                            cand[w * WW + dy * W + dx] =
+                            const unsigned long long key =
                                 member_of(w, y, x)
                                     ? (static_cast<unsigned long long>(dist_key(a)) << 32) | pack_pos(0, y, x)
                                     : ~0ull;
+                            if (held)
+                                strip[q] = key;
+                            else
+                                cand[w * WW + dy * W + dx] = key;
                         }
                     }
                 }
             }
             int nb = 0;
-            for (int base = 0; base < cells; base += tab.chunk) {
+            for (; held && nb < kl; ++nb) {
+                const unsigned long long m = min(strip[0], min(strip[1], strip[2]));
+                const uint32_t d = static_cast<uint32_t>(m >> 32), at = static_cast<uint32_t>(m);
+                const uint32_t mn = wave_min_u32_dpp(d);
+                if (mn == kTaken) break;  // no member left
+                const unsigned long long who = __builtin_amdgcn_ballot_w64(d == mn);
+                uint32_t first = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(at), __builtin_ctzll(who)));
+                if ((who & (who - 1u)) != 0) first = wave_min_u32_dpp(d == mn ? at : ~0u);  // equal distances
+                const unsigned long long win = (static_cast<unsigned long long>(mn) << 32) | first;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) strip[q] = strip[q] == win ? ~0ull : strip[q];
+                if (lane == 0) best[nb] = win;
+            }
+            if (held) __syncthreads();
+            for (int base = 0; base < cells && !held; base += tab.chunk) {
                 const int cnt = min(tab.chunk, cells - base);
                 for (int c = lane; c < cnt && !staged; c += 64) {
                     const int cell = base + c;
