@@ -799,9 +799,10 @@ __global__ __launch_bounds__(64) void match_wave_kernel(MatchTable tab) {
 // carry (non-finite, or |v - mu| >= 8192 so that S would be negative) or
 // nothing but one value, scores its whole window exactly.
 //
-// What bounds it: VALU issue (per wave of the step-3, range-16, group-16
-// launch 3.8 k instructions before the row scoring against 6.0 k with the
-// norms, masks and rank sums on the VALU) and LDS reads of the scoring. Per
+// What bounds it: VALU issue and the matrix unit together (per wave of the
+// step-3, range-16, group-16 launch 3.05 k VALU instructions against 6.0 k with
+// the norms, masks and rank sums on the VALU, and 186 MFMAs; about 80 % of the
+// SIMDs' cycles; the passes take 60 % of the time). Per
 // 1080p YUV420 frame at step 3, range 16: group 16 on the noisy planes 660 us
 // (1115 before the norms and masks went into the MFMAs, the sums of ranks into
 // row minima and the reference's patch into registers), group 32 on the
