@@ -1,6 +1,7 @@
 """Builds tests/asan/capi_stress: the library's sources and the C ABI driver
 with AddressSanitizer on the host code only (the device code of every .hip
-file is built as in the product), linked into one executable.
+file is built as in the product), linked into one executable; and plan_sizes,
+the same sources with the driver of the plans' sizes.
 
     python tests/asan/build_asan.py
 
@@ -17,6 +18,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(os.path.dirname(HERE))
 PKG = os.path.join(ROOT, "vapoursynth-nssfactory_amd")
 EXE = os.path.join(HERE, "capi_stress")
+PLAN_EXE = os.path.join(HERE, "plan_sizes")
 
 _spec = importlib.util.spec_from_file_location("nss_build", os.path.join(PKG, "build.py"))
 _pkg_build = importlib.util.module_from_spec(_spec)
@@ -34,7 +36,7 @@ def build(jobs: int = 4) -> str:
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     flags = [f for f in _pkg_build.HIPFLAGS if f != "-O3"] + ["-O1", "-g"]
     units = [(os.path.join(PKG, "csrc", s), s.endswith(".hip")) for s in _pkg_build.SOURCES]
-    units.append((os.path.join(HERE, "capi_stress.cpp"), False))
+    units += [(os.path.join(HERE, os.path.basename(exe) + ".cpp"), False) for exe in (EXE, PLAN_EXE)]
     objs, procs = [], []
     for src, is_hip in units:
         obj = os.path.join(objdir, os.path.splitext(os.path.basename(src))[0] + ".o")
@@ -48,11 +50,13 @@ def build(jobs: int = 4) -> str:
         if p.wait() != 0:
             raise subprocess.CalledProcessError(1, "hipcc")
     clang = "/opt/rocm/llvm/bin/clang++"
-    link = [clang, *LINK_ASAN, "-o", EXE + ".tmp", *objs, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib",
-            "-lpthread"]
-    print(" ".join(link), flush=True)
-    subprocess.check_call(link)
-    os.replace(EXE + ".tmp", EXE)
+    drivers = objs[-2:]
+    for exe, driver in zip((EXE, PLAN_EXE), drivers):
+        link = [clang, *LINK_ASAN, "-o", exe + ".tmp", *objs[:-2], driver, "-L/opt/rocm/lib", "-lamdhip64",
+                "-Wl,-rpath,/opt/rocm/lib", "-lpthread"]
+        print(" ".join(link), flush=True)
+        subprocess.check_call(link)
+        os.replace(exe + ".tmp", exe)
     return EXE
 
 

@@ -4714,12 +4714,14 @@ inline constexpr size_t kMmStagedLds = 40 * 1024;
 
 // LDS words of the MFMA matcher for `list` candidates per reference: the fp16
 // region (the exact keys over it), the exchange and lists, counters, and with
-// `staged` the FP32 region.
+// `staged` the FP32 region. Plans ask for every block size: unions wider than
+// the pitch table (steps above 8 only) get a size that no LDS holds.
 static size_t mm_lds_words(int step, int range, size_t list, bool staged) {
     // the union of a 4 x 4 block's windows spans at most 3 step + 2 range + 1
     // candidate columns and rows
     const int span = 3 * step + 2 * range + 1;
     const int nt = (span + 15) >> 4;
+    if (nt > kMmTiles) return size_t{1} << 20;
     const size_t reg = (std::max(static_cast<size_t>(span + 7) * static_cast<size_t>(h_mm_pitch.of[nt]), 16 * list) + 3) & ~static_cast<size_t>(3);
     return reg + 8 * list + kMmCounters +
            (staged ? static_cast<size_t>(span + 7) * mm_pitch32(nt) : 0);
@@ -4736,7 +4738,7 @@ size_t match_mfma_lds_bytes(int step, int range, int group) {
 }
 
 bool match_mfma_fits(int block, int group, int step, int range, int width, int height) {
-    return block == 8 && group >= 1 && group <= 32 && width >= 8 && height >= 8 && 3 * step + 2 * range + 1 <= 16 * kMmTiles &&
+    return block == 8 && group >= 1 && group <= 32 && width >= 8 && height >= 8 &&
            match_mfma_lds_bytes(step, range, group) <= 160 * 1024;
 }
 
