@@ -1818,9 +1818,11 @@ __device__ __forceinline__ void to_fixed_n(const float (&v)[N], unsigned long lo
     }
 }
 
-// n / d, correctly rounded, for d in [2^-60, 2^62] and 0 <= n <= d: Newton's
-// step on the reciprocal and two residual corrections (the operations of the
-// full division without its scaling and special cases).
+// n / d for d in [2^-60, 2^62] and 0 <= n <= d: Newton's step on the reciprocal
+// and two residual corrections (the operations of the full division without
+// its scaling and special cases). Correctly rounded for n = 0 and n >= 2^-101;
+// below that (quotients below 2^-41) the residuals underflow and the last
+// place may be off.
 __device__ __forceinline__ float quotient(float n, float d) {
     float y = __builtin_amdgcn_rcpf(d);
     y = fmaf(fmaf(-d, y, 1.f), y, y);
@@ -1831,6 +1833,9 @@ __device__ __forceinline__ float quotient(float n, float d) {
 
 // Wiener gains r^2 / (r^2 + sig2) applied to a lane's G coefficients (lane 0's
 // first, the group's mean, keeps 1); the sum of their squares is returned.
+// quotient() serves coefficients below 2^30 and sig2 in (2^-60, 2^61), so that
+// the denominators stay in its range; any finite sigma is accepted, and its
+// square may be infinite (gain 0).
 template <int G>
 __device__ __forceinline__ float wiener_shrink(float (&c)[G], const float (&r)[G], float sig2, int lane) {
     float mag = 0.f, w2 = 0.f;
@@ -1848,7 +1853,7 @@ __device__ __forceinline__ float wiener_shrink(float (&c)[G], const float (&r)[G
             w2 = fmaf(w, w, w2);
         }
     };
-    if (mag < 1073741824.f && sig2 > 0x1p-60f)
+    if (mag < 1073741824.f && sig2 > 0x1p-60f && sig2 < 0x1p61f)
         shrink([](float n, float d) { return quotient(n, d); });
     else
         shrink([](float n, float d) { return d > 0.f ? n / d : 0.f; });
