@@ -796,8 +796,8 @@ __global__ __launch_bounds__(64) void match_wave_kernel(MatchTable tab) {
 // matchers (rows, then columns, one fmaf per pixel) and taken in order of
 // (dist, y, x): the records are those of match_run_kernel bit for bit. A
 // reference whose list overflows, or a block holding a value fp16 cannot
-// carry (non-finite, or |v - mu| >= 8192 so that S would be negative) or
-// nothing but one value, scores its whole window exactly.
+// carry (non-finite, or |v - mu| >= 8192 so that S would be negative), scores
+// its whole window exactly. A region of one value needs no scores at all.
 //
 // What bounds it: VALU issue and the matrix unit together (per wave of the
 // step-3, range-16, group-16 launch 3.05 k VALU instructions against 6.0 k with
@@ -1159,12 +1159,33 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
     __syncthreads();
     const uint32_t bmax_bits = __builtin_amdgcn_readfirstlane(row_max_u32(xw[n]));
     const float bmax = __uint_as_float(bmax_bits) * (1.f / 4096.f);
-    bool anybad = bmax_bits >= kNonFinite || !(bmax < 8192.f);
+    // One value everywhere (mu is then exactly it, and no difference vanishes
+    // in the scaling): every distance is 0, so the records are the first places
+    // of the window, the reference's own left out. Lane n of row g of wave w
+    // takes the records n + 1, n + 17 of reference 4 w + g. Scoring the windows
+    // of such regions exactly cost more than the run matcher does: 1080p, group
+    // 16, half the frame constant: step 3, range 9 452 -> 281 us (run matcher
+    // 341); step 4, range 9 252 -> 141 (196).
+    const bool flat_region = bmax_bits == 0u;
+    if (flat_region) {
+        const int m = 4 * wave + g, K = kmv[m];
+        const int ri = i0 + min(m >> 2, ncol - 1), rj = j0 + min(m & 3, nrow - 1);
+        const MmWin w = mm_win(jb, ri, rj);
+        const int ww = w.right - w.left + 1, self = (w.cy - w.top) * ww + (w.cx - w.left);
+        const float inv_ww = 1.f / static_cast<float>(ww);
+        MatchRec* out = jb.out + (static_cast<size_t>(rj) * jb.grid.nx + ri) * G + 1;
+        for (int k = n; k < K; k += 16) {
+            const int c = k + (k >= self ? 1 : 0);
+            const int dy = div_small(c, inv_ww), dx = c - dy * ww;
+            out[k] = MatchRec{w.left + dx, w.top + dy, jb.t0, 0u};
+        }
+    }
+    bool anybad = bmax_bits >= kNonFinite || !(bmax < 8192.f) || flat_region;
     if (!anybad && !(bmax >= 0.015625f && bmax < 2.f)) {
         int ex = 0;
         (void)frexpf(bmax, &ex);
         const int S = min(13 - ex, 40);
-        anybad = S < 0 || bmax == 0.f;  // a constant region: every candidate would be listed
+        anybad = S < 0;
         if (!anybad) {
             const float sc = ldexpf(1.f, S), msc = -mu * sc;
             each_word([&](int yy, int w, float v0, float v1) {
@@ -1473,6 +1494,7 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
         jb.counts[ref_id] = 1 + kmv[tid];
     }
 
+    if (flat_region) return;
     // (no reference of the block needs the rest: the usual case)
     if (__builtin_amdgcn_ballot_w64(kmv[n] > 0 && (anybad || cnt[n] > LIST)) == 0) return;
     __syncthreads();  // the regions and lists become the fallback's keys
