@@ -53,7 +53,7 @@ int match_workgroups(int kind, const Grid& g);
 // FP32 matchers only, 2 the MFMA matcher wherever it fits.
 int match_path();
 // Automatic choice: the MFMA matcher also where the run matcher fits, when
-// the window is wide against the step and the stage has references enough.
+// the stage has references enough for the window and the step.
 bool match_mfma_pays(int step, int range, int group, long long nref);
 size_t filter_atomic_lds_bytes(int block, int group, bool wiener);
 size_t filter_tile_lds_bytes(int block, int group, bool wiener, const TileGeom& t);
