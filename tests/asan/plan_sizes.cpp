@@ -4,14 +4,25 @@
 //   plan_sizes                      sizes every allowed block, step, range and group
 //   plan_sizes S R G W H N ...      the matcher kind chosen for each six numbers: block 8,
 //                                   step S, range R, group G, W x H planes, N references
+//   plan_sizes tiles G S R N ...    the group filters' tile for each four numbers: group G,
+//                                   step S, range R, N references ("0 0": the atomic path)
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 
 #include "../../vapoursynth-nssfactory_amd/csrc/instance.hpp"
 
 using namespace nsship;
 
 int main(int argc, char** argv) {
+    if (argc > 1 && !std::strcmp(argv[1], "tiles")) {
+        for (int i = 2; i + 3 < argc; i += 4) {
+            const TileShape t = gram_tile_shape(8, std::atoi(argv[i]), std::atoi(argv[i + 1]), std::atoi(argv[i + 2]),
+                                                std::atoll(argv[i + 3]));
+            std::printf("%d %d\n", t.tw, t.th);
+        }
+        return 0;
+    }
     if (argc > 1) {
         for (int i = 1; i + 5 < argc; i += 6) {
             int v[6];

@@ -1,7 +1,8 @@
 """Sizes and matcher choices of the plans on the CPU (tests/asan/plan_sizes: the
 library's sources with AddressSanitizer on the host code): every allowed block,
 step, range and group is sized without a read outside a table, and the automatic
-choice of the matcher of block 8 on both sides of each of its lines."""
+choice of the matcher of block 8 and of the group filters' tiles on both sides
+of each of its lines."""
 import os
 import subprocess
 import sys
@@ -53,3 +54,27 @@ def test_matcher_choice(plan_sizes, kind, step, rng, group, refs):
     r = plan_sizes(step, rng, group, 1920, 1080, refs)
     assert r.returncode == 0, r.stderr[-2000:]
     assert int(r.stdout) == kind
+
+
+def _over(tw, th, step, rng):
+    """Tiles over a pixel: (accumulation rectangle, pixels from tile to tile)."""
+    return ((tw - 1) * step + 2 * rng + 8) * ((th - 1) * step + 2 * rng + 8), tw * th * step * step
+
+
+# the smallest launch of each shape's tiles, and one reference less; groups of 8
+# leave the tiles where only 4 x 2 of them fit, groups of 16 where none do
+@pytest.mark.parametrize("group,step,rng,tw,th,least", [
+    (8, 8, 7, 8, 4, 2048), (8, 8, 27, 8, 4, 2048), (8, 2, 20, 8, 4, 100), (8, 1, 24, 8, 4, 100), (8, 1, 44, 8, 4, 100),
+    (8, 8, 28, 4, 4, 480), (8, 8, 34, 4, 4, 480), (8, 4, 40, 4, 4, 480), (8, 2, 42, 4, 4, 480),
+    (8, 8, 35, 0, 0, 0), (8, 4, 42, 0, 0, 0), (8, 2, 44, 0, 0, 0), (8, 8, 39, 0, 0, 0),
+    (16, 8, 7, 4, 4, 30), (16, 1, 34, 4, 4, 30), (16, 8, 34, 4, 4, 30), (16, 8, 35, 4, 2, 30), (16, 2, 44, 4, 2, 30),
+    (16, 8, 40, 0, 0, 0), (32, 8, 7, 0, 0, 0), (4, 8, 7, 0, 0, 0)])
+def test_group_filter_tiles(plan_sizes, group, step, rng, tw, th, least):
+    if not tw:
+        r = plan_sizes("tiles", group, step, rng, 1 << 24)
+        assert r.stdout == "0 0\n", r.stdout + r.stderr[-2000:]
+        return
+    area, pitch = _over(tw, th, step, rng)
+    refs = least if least == 2048 else -(-least * area // pitch)
+    r = plan_sizes("tiles", group, step, rng, refs, group, step, rng, refs - 1)
+    assert r.stdout == f"{tw} {th}\n0 0\n", r.stdout + r.stderr[-2000:]

@@ -78,8 +78,13 @@ size_t wnnm_lds_bytes(int block, int group);
 // ncsr: the NCSR code shrink on the same eigenbasis instead of WNNM's.
 hipError_t launch_wnnm(const WnnmTable& t, int total_wg, bool ncsr, hipStream_t s);
 // The same on tiles of references, for full groups of 8 or 16 blocks of 8 of
-// spatial planes: LDS bytes of a plane's tiles (0 where it does not serve the
-// shape) and the launch.
+// spatial planes: the references of a tile for a launch of nref in all (0 x 0
+// where the atomic path serves better), LDS bytes of a plane's tiles (0 where
+// the kernel does not serve the shape) and the launch.
+struct TileShape {
+    int tw, th;
+};
+TileShape gram_tile_shape(int block, int group, int step, int range, long long nref);
 size_t gram_tile_lds_bytes(int block, int group, int range, int width, int height, const TileGeom& g);
 hipError_t launch_wnnm_tiles(const WnnmTable& t, int total_wg, size_t lds, bool ncsr, hipStream_t s);
 hipError_t launch_regularize(float* est, int est_stride, const float* noisy, int noisy_stride, int width, int height,

@@ -15,11 +15,42 @@
 #include <mutex>
 #include <new>
 #include <string>
-#include <utility>
 
 #include "instance.hpp"
 
 using namespace nsship;
+
+// The largest tile whose sums leave two workgroups per CU, if the launch has
+// the references for it. A tile of groups of 8 fills the kernel's four waves
+// at 8 x 4 references, one of groups of 16 at 4 x 4; the finish reads, for
+// every pixel, each tile that reaches it (`over` of them: the tile's rectangle
+// in steps of tiles), and a launch of few references is mostly that and the
+// tiles' own latency. Atomic path's time over the tile path's, WNNM (NCSR is
+// alike), steps 1 to 8, ranges 2 to 48:
+//   groups of 8, 8 x 4: 1080p 1.65 to 2.95, 640 x 480 1.15 to 3.7; 1 to 1.7
+//     from 2048 references and 100 for each tile over a pixel on, below that
+//     0.78 to 1.03 (128 x 96 at step 8, range 16 0.95, at step 1, range 40
+//     0.78; 256 x 256 at step 8, range 24 0.97) but for 1.07 to 1.18 near it;
+//   groups of 8, 4 x 4 (two waves idle): 1080p 1.07 to 1.65, 640 x 480 1.0 to
+//     1.5 from 480 per tile on; 256 x 256 0.90 to 1.04, 128 x 96 0.74 to 0.94;
+//   groups of 8, 4 x 2 (three idle): 0.63 to 0.91, so never;
+//   groups of 16, 4 x 4: 1080p 2.0 to 3.8, 640 x 480 1.5 to 3.9, 256 x 256 1.2
+//     to 3.5, 128 x 96 1.0 to 2.4; 0.83 to 1.03 below 30 per tile (128 x 96,
+//     step 1, from range 34 on); 4 x 2: 1.1 to 1.4, 0.72 below (128 x 96).
+TileShape nsship::gram_tile_shape(int block, int group, int step, int range, long long nref) {
+    if (block != 8 || (group != 8 && group != 16)) return TileShape{0, 0};
+    for (const TileShape sh : {TileShape{8, 4}, TileShape{4, 4}, TileShape{4, 2}}) {
+        const TileGeom g = make_tiles(Grid{1, 1, step}, sh.tw, sh.th, block, range);
+        const size_t lds = gram_tile_lds_bytes(block, group, range, 1 << 20, 1 << 20, g);
+        if (lds == 0 || lds > kTileLdsBudget) continue;
+        const long long per = group == 16 ? 30 : sh.tw == 8 ? 100 : 480;
+        if (group == 8 && (sh.th == 2 || nref < 2048)) break;
+        // nref >= per * over
+        if (nref * sh.tw * sh.th * step * step < per * g.aw * g.ah) break;
+        return sh;
+    }
+    return TileShape{0, 0};
+}
 
 struct nss_hip_wnnm {
     nss_hip_wnnm_params p{};
@@ -77,31 +108,25 @@ void release(nss_hip_wnnm* h) {
     }
 }
 
-// The tile path's plan (radius 0), when it serves every active plane: the
-// largest tile whose sums leave two workgroups per CU, in shapes that fill the
-// kernel's four waves (64 / group groups each). 1080p, groups of 8 at range 7:
-// 8 x 4 references 59 us; 4 x 4, two waves of each workgroup idle, 83 us.
+// The tile path's plan (radius 0), when it serves every active plane.
 bool plan_tiles(nss_hip_wnnm* h) {
     const nss_hip_wnnm_params& p = h->p;
-    const int per_tile = 4 * (64 / std::max(p.group_size, 1));
-    for (const auto& sh : {std::pair<int, int>{8, 4}, {4, 4}, {4, 2}}) {
-        if (p.radius > 0 || sh.first * sh.second > per_tile) continue;
-        size_t lds = 0;
-        bool ok = true;
-        for (int i = 0; i < h->vi.num_planes; ++i) {
-            auto& q = h->pl[i];
-            if (!q.active) continue;
-            q.tiles = make_tiles(q.grid, sh.first, sh.second, p.block_size, p.bm_range);
-            const size_t need =
-                gram_tile_lds_bytes(p.block_size, p.group_size, p.bm_range, q.width, q.height, q.tiles);
-            ok &= need != 0;
-            lds = std::max(lds, need);
-        }
-        if (!ok || lds > kTileLdsBudget) continue;
-        h->tile_lds = lds;
-        return true;
+    if (p.radius > 0) return false;
+    long long nref = 0;
+    for (const auto& q : h->pl) nref += q.active ? q.nref : 0;
+    const TileShape sh = gram_tile_shape(p.block_size, p.group_size, p.block_step, p.bm_range, nref);
+    if (!sh.tw) return false;
+    size_t lds = 0;
+    for (int i = 0; i < h->vi.num_planes; ++i) {
+        auto& q = h->pl[i];
+        if (!q.active) continue;
+        q.tiles = make_tiles(q.grid, sh.tw, sh.th, p.block_size, p.bm_range);
+        const size_t need = gram_tile_lds_bytes(p.block_size, p.group_size, p.bm_range, q.width, q.height, q.tiles);
+        if (!need) return false;
+        lds = std::max(lds, need);
     }
-    return false;
+    h->tile_lds = lds;
+    return true;
 }
 
 // Buffers of every active plane; h->ncsr and the parameters are set.
