@@ -204,21 +204,37 @@ int init_instance(nss_hip_wnnm* h, const nss_hip_wnnm_params& p, const nss_hip_v
         return fail(NSS_HIP_INVALID_INPUT, ns + ": memory_limit_mb is too small for this clip: the instance needs at "
                                                 "least " + std::to_string(need) + " MiB");
     }
-    for (int i = 0; i < info->num_planes; ++i) {
-        auto& q = h->pl[i];
-        if (!q.active) continue;
-        size_t z[7];
-        sizes(q, z);
-        q.part_elems = z[3] ? z[3] / sizeof(unsigned long long) - q.nref : 0;
-        if ((e = dev_alloc(&q.recs, z[0])) != hipSuccess || (e = dev_alloc(&q.counts, z[1])) != hipSuccess ||
-            (z[2] && ((e = dev_alloc(&q.num, z[2] / 2)) != hipSuccess || (e = dev_alloc(&q.den, z[2] / 2)) != hipSuccess)) ||
-            (z[3] && (e = dev_alloc(&q.part, z[3])) != hipSuccess) || (z[4] && (e = dev_alloc(&q.est, z[4])) != hipSuccess) ||
-            (z[5] && (e = dev_alloc(&q.win, z[5])) != hipSuccess) ||
-            (z[6] && (e = dev_alloc(&q.mwin, z[6])) != hipSuccess)) {
-            release(h);
-            return hip_fail(e, "group filter buffers");
+    auto allocate = [&]() {
+        for (int i = 0; i < info->num_planes; ++i) {
+            auto& q = h->pl[i];
+            if (!q.active) continue;
+            size_t z[7];
+            sizes(q, z);
+            q.part_elems = z[3] ? z[3] / sizeof(unsigned long long) - q.nref : 0;
+            if ((e = dev_alloc(&q.recs, z[0])) != hipSuccess || (e = dev_alloc(&q.counts, z[1])) != hipSuccess ||
+                (z[2] &&
+                 ((e = dev_alloc(&q.num, z[2] / 2)) != hipSuccess || (e = dev_alloc(&q.den, z[2] / 2)) != hipSuccess)) ||
+                (z[3] && (e = dev_alloc(&q.part, z[3])) != hipSuccess) ||
+                (z[4] && (e = dev_alloc(&q.est, z[4])) != hipSuccess) ||
+                (z[5] && (e = dev_alloc(&q.win, z[5])) != hipSuccess) ||
+                (z[6] && (e = dev_alloc(&q.mwin, z[6])) != hipSuccess)) {
+                release(h);
+                return e;
+            }
         }
+        return hipSuccess;
+    };
+    e = allocate();
+    if (e != hipSuccess && h->tiled) {
+        // A device too full for the tiles' partials (up to 30 times the sums
+        // at step 1) may still hold the atomic path's sums.
+        const long long tile_bytes = h->bytes;
+        (void)hipGetLastError();
+        h->tiled = false;
+        h->bytes = total();
+        if (h->bytes < tile_bytes) e = allocate();
     }
+    if (e != hipSuccess) return hip_fail(e, "group filter buffers");
     return NSS_HIP_OK;
 }
 
