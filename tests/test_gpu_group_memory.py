@@ -1,5 +1,9 @@
 """WNNM and NCSR instances on a device without room for the tiles' partials: the
-atomic path's smaller sums are allocated instead, with the same output."""
+atomic path's smaller sums are allocated instead, with the same output. And a
+refused memory limit names the least one that is accepted, whichever of the two
+paths it is for."""
+import re
+
 import numpy as np
 import pytest
 
@@ -42,3 +46,17 @@ def test_a_failed_allocation_of_the_tile_path(gpu, kind, allocations, group):
             assert gpu.debug_live_allocations() == base
     finally:
         gpu.debug_fail_alloc(-1)
+
+
+@pytest.mark.parametrize("kind", ["WNNM", "NCSR"])
+@pytest.mark.parametrize("kw", [dict(block_step=8, bm_range=5), dict(block_step=4, bm_range=9),
+                                dict(block_step=8, bm_range=9, group_size=32)])
+def test_a_refused_limit_names_the_least(gpu, kind, kw):
+    # at step 8 and range 5 the partials are the smaller buffer, else the sums
+    make = getattr(gpu, kind)
+    with pytest.raises(gpu.Error, match="memory_limit_mb is too small") as e:
+        make("GRAYS", 1920, 1080, sigma=[10.0], memory_limit_mb=1, **kw)
+    least = int(re.search(r"at least (\d+) MiB", str(e.value)).group(1))
+    make("GRAYS", 1920, 1080, sigma=[10.0], memory_limit_mb=least, **kw).close()
+    with pytest.raises(gpu.Error, match="memory_limit_mb is too small"):
+        make("GRAYS", 1920, 1080, sigma=[10.0], memory_limit_mb=least - 1, **kw)

@@ -195,12 +195,14 @@ int init_instance(nss_hip_wnnm* h, const nss_hip_wnnm_params& p, const nss_hip_v
     const long long limit = p.memory_limit_mb > 0 ? static_cast<long long>(p.memory_limit_mb) << 20 : 0;
     h->tiled = plan_tiles(h);
     h->bytes = total();
+    long long least = h->bytes;
     if (h->tiled && limit && h->bytes > limit) {
         h->tiled = false;
         h->bytes = total();
+        least = std::min(least, h->bytes);
     }
     if (limit && h->bytes > limit) {
-        const long long need = (h->bytes + (1ll << 20) - 1) >> 20;
+        const long long need = (least + (1ll << 20) - 1) >> 20;
         return fail(NSS_HIP_INVALID_INPUT, ns + ": memory_limit_mb is too small for this clip: the instance needs at "
                                                 "least " + std::to_string(need) + " MiB");
     }
