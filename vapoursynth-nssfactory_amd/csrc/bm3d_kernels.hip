@@ -2174,8 +2174,8 @@ __device__ inline void gather_rows_b8(const float* plane, int stride, const Matc
 
 // Tile kernel for block 8: LDS = num [ah][aw] int64 | match records of the
 // tile | per-wave transpose buffers.
-template <int G, bool WIENER>
-__global__ __launch_bounds__(G <= 16 ? 1024 : 256) void filter_tile_b8_kernel(FilterTable tab) {
+template <int G, bool WIENER, int MAXW>
+__global__ __launch_bounds__(64 * MAXW) void filter_tile_b8_kernel(FilterTable tab) {
     extern __shared__ __align__(16) unsigned long long acc[];
     constexpr int B = 8;
     constexpr int M = G / 8;
@@ -4961,13 +4961,18 @@ static hipError_t launch_filter_b(const FilterTable& t, int total_wg, size_t lds
 // A launch of up to 256 workgroups has a CU for each: 16 waves share a filter
 // tile's groups, and the finish takes one pixel per thread. 128 x 96 YUV420,
 // group 8: hard 10.8 -> 7.1 us, Wiener 12.5 -> 8.4; finish of 256 x 256 at step
-// 3, group 16: 22.7 -> 19.6. Above that, eight waves per tile serve the hard
-// stage (1080p YUV420 43.5 -> 42.0 us, 256 x 256 at step 3, group 16 18.6 ->
-// 16.8) and four the Wiener stage (57.3 us against 60.8: its registers leave
-// the fifth to eighth wave of a SIMD out).
+// 3, group 16: 22.7 -> 19.6. Above that four waves serve the Wiener stage
+// (1080p YUV420 57.3 us against 60.8 with eight: its registers leave the fifth
+// to eighth wave of a SIMD out), and eight the hard stage where they put a
+// fifth more waves on a CU than workgroups of four do, or where the tiles fill
+// the device no more than twice. Eight against four, 1080p, group 8: step 8, range 9
+// 28.4 us against 29.3, range 24 47.1 / 55.3, step 6, range 24 61.6 / 78.8; RGB,
+// step 3, range 7 (28 waves to 32) 397 / 374; group 16: step 3, range 24 309 /
+// 398, but range 12 (16 waves either way) 271 / 255. Each form is compiled for
+// its own size: one bound of 1024 threads for all of them took group 16's hard
+// kernel from 71 to 86 registers (RGB, step 3, range 4: 711 -> 790 us).
 inline constexpr int kFinishAloneBlocks = 256;
 inline constexpr int kFilterAloneTiles = 256;
-inline constexpr int kFilterWaves = 8;
 
 template <int G>
 static hipError_t launch_filter_b8(const FilterTable& t, int total_wg, size_t lds, bool wiener, hipStream_t s) {
@@ -4976,7 +4981,14 @@ static hipError_t launch_filter_b8(const FilterTable& t, int total_wg, size_t ld
         const size_t each = static_cast<size_t>(G) * kTs * 4;
         int groups = 1;
         for (int j = 0; j < t.n; ++j) groups = std::max(groups, t.job[j].tiles.tw * t.job[j].tiles.th);
-        const int want = total_wg <= kFilterAloneTiles ? 16 : wiener ? 4 : kFilterWaves;
+        // waves of a CU with workgroups of w (LDS comes in units of 1280 bytes;
+        // group 16's registers hold 24)
+        const auto per_cu = [&](int w) {
+            const size_t units = (lds + (w - 4) * each + 1279) / 1280;
+            return std::min(G <= 8 ? 32 : 24, w * static_cast<int>(128 / units));
+        };
+        const bool eight = !wiener && (5 * per_cu(8) >= 6 * per_cu(4) || total_wg <= 2 * 64 * per_cu(4));
+        const int want = total_wg <= kFilterAloneTiles ? 16 : eight ? 8 : 4;
         while (2 * waves <= want && waves < groups && lds + waves * each <= (want == 16 ? 160 : 80) * 1024) {
             lds += waves * each;
             waves *= 2;
@@ -4985,12 +4997,14 @@ static hipError_t launch_filter_b8(const FilterTable& t, int total_wg, size_t ld
     const auto launch = [&](auto kernel) {
         allow_lds(kernel, lds);
         kernel<<<total_wg, 64 * waves, lds, s>>>(t);
+        return hipGetLastError();
     };
-    if (wiener)
-        launch(&filter_tile_b8_kernel<G, true>);
-    else
-        launch(&filter_tile_b8_kernel<G, false>);
-    return hipGetLastError();
+    if constexpr (G <= 16) {
+        if (wiener && waves > 4) return launch(&filter_tile_b8_kernel<G, true, 16>);
+        if (!wiener && waves > 8) return launch(&filter_tile_b8_kernel<G, false, 16>);
+        if (!wiener && waves > 4) return launch(&filter_tile_b8_kernel<G, false, 8>);
+    }
+    return wiener ? launch(&filter_tile_b8_kernel<G, true, 4>) : launch(&filter_tile_b8_kernel<G, false, 4>);
 }
 
 template <int G, int FORM>
