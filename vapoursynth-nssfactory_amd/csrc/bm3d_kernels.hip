@@ -1164,8 +1164,8 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
     // of the window, the reference's own left out. Lane n of row g of wave w
     // takes the records n + 1, n + 17 of reference 4 w + g. Scoring the windows
     // of such regions exactly cost more than the run matcher does: 1080p, group
-    // 16, half the frame constant: step 3, range 9 452 -> 281 us (run matcher
-    // 341); step 4, range 9 252 -> 141 (196).
+    // 16, half the frame constant: step 3, range 9 452 us (run matcher 341), now
+    // 236; step 4, range 9 252 (196), now 127.
     const bool flat_region = bmax_bits == 0u;
     if (flat_region) {
         const int m = 4 * wave + g, K = kmv[m];
@@ -1503,8 +1503,12 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
     // per thread) into LDS, then a wave per reference takes the G - 1 smallest
     // by rounds of a wave minimum over each lane's four best. Windows that do
     // not fit come in pieces; the lanes carry the best so far. A window whose
-    // first 256 places hold G - 1 copies of the patch (distance 0) is done with
-    // those: no later place can displace one (flat areas).
+    // first places hold G - 1 copies of the patch (distance 0) is done with
+    // those: no later place can displace one (flat areas). A wave looks through
+    // the first 64 of its own reference's, then all four through each other
+    // reference's next 256: against 256 by all at once, 1080p at step 3, range 7,
+    // group 8: half the frame constant 239 -> 181 us, squares of 100 pixels 450
+    // -> 310.
     const int space = reg_words + kUnion;
     const int wcap = min((2 * jb.range + 1) * (2 * jb.range + 1), (ux1 - ux0 + 1) * (uy1 - uy0 + 1));
     const int at_once = max(1, min(4, space / wcap));
@@ -1520,9 +1524,10 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
         if (tid < 4) copies[tid] = 0;
         __syncthreads();
         unsigned long long kept = ~0ull;  // lane k: the k-th best of the pieces so far
-        uint32_t flat = 0u;               // the references done after 256 places, a bit each
-        // keys of places from .. to - 1 (p0 the piece's first) of the r-th reference
-        auto score = [&](int r, int p0, int from, int to) {
+        uint32_t flat = 0u;               // the references done after their first places, a bit each
+        // keys of places from .. to - 1 (p0 the piece's first) of the r-th
+        // reference, by one wave or by all four; returns the copies found
+        auto score = [&](int r, int p0, int from, int to, bool alone) {
             const int m = (refs >> (4 * r)) & 15;
             const MmWin w = mm_win(jb, i0 + (m >> 2), j0 + (m & 3));
             const int ww = w.right - w.left + 1, end = min(ww * (w.bottom - w.top + 1), to);
@@ -1531,7 +1536,8 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
             float patch[4];
             row_patch(w.cx, w.cy, patch);
             int zeros = 0;
-            for (int q0 = from + 64 * wave; q0 < end; q0 += 256) {
+            const int by = alone ? 64 : 256;
+            for (int q0 = from + (alone ? 0 : 64 * wave); q0 < end; q0 += by) {
                 const int c = min(q0 + lane, end - 1);
                 const int dy = div_small(c, inv_ww), dx = c - dy * ww;
                 const uint32_t d = exact(patch, w.left - ux0 + dx, w.top - uy0 + dy);
@@ -1551,18 +1557,26 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
         for (int p0 = 0; p0 < wcap && flat != (1u << nref) - 1u; p0 += piece) {
             int from = p0;
             if (p0 == 0) {
-                from = min(piece, 256);
-                for (int r = 0; r < nref; ++r) {
-                    const int zeros = score(r, 0, 0, from);
-                    if (lane == 0) atomicAdd(&copies[r], zeros);
+                // (a reference done after 64 places has its copies among them:
+                // its keys from there to `from` are not written and not read)
+                for (int pass = 0; pass < 2 && flat != (1u << nref) - 1u; ++pass) {
+                    const int next = min(piece, pass == 0 ? 64 : 320);
+                    for (int r = 0; r < nref; ++r)
+                        if (pass == 0 ? r == wave : !((flat >> r) & 1u)) {
+                            const int zeros = score(r, 0, from, next, pass == 0);
+                            if (lane == 0) atomicAdd(&copies[r], zeros);
+                        }
+                    from = next;
+                    __syncthreads();
+                    for (int r = 0; r < nref; ++r)
+                        flat |= copies[r] >= kmv[(refs >> (4 * r)) & 15] ? 1u << r : 0u;
+                    flat = __builtin_amdgcn_readfirstlane(flat);
+                    __syncthreads();
                 }
-                __syncthreads();
-                for (int r = 0; r < nref; ++r)
-                    flat |= copies[r] >= kmv[(refs >> (4 * r)) & 15] ? 1u << r : 0u;
             }
             const uint32_t skip = __builtin_amdgcn_readfirstlane(flat);
             for (int r = 0; r < nref; ++r)
-                if (!((skip >> r) & 1u)) score(r, p0, from, p0 + piece);
+                if (!((skip >> r) & 1u)) score(r, p0, from, p0 + piece, false);
             __syncthreads();
             const bool copied = (skip >> wave) & 1u;
             const int m = wave < nref ? (refs >> (4 * wave)) & 15 : 0;
