@@ -37,16 +37,18 @@ MFMA, RUN, WAVE = 3, 2, 1
 
 
 @pytest.mark.parametrize("kind,step,rng,group,refs", [
-    # ranges up to 5: steps up to 4, groups up to 16, 49152 references
+    # ranges up to 9: steps up to 4, groups up to 16, 49152 references (16384 for
+    # ranges up to 4 at groups up to 8)
+    (RUN, 4, 4, 8, 16383), (MFMA, 4, 4, 8, 16384), (RUN, 4, 5, 8, 49151), (MFMA, 4, 5, 8, 49152),
     (MFMA, 1, 1, 16, 49152), (RUN, 1, 1, 16, 49151), (MFMA, 4, 5, 16, 49152), (RUN, 4, 5, 16, 49151),
-    (RUN, 5, 5, 8, 1 << 20), (RUN, 4, 5, 32, 1 << 20),
-    # ranges 6 to 9: 98304
-    (RUN, 4, 6, 8, 98303), (MFMA, 4, 6, 8, 98304), (RUN, 3, 9, 16, 98303), (MFMA, 3, 9, 16, 98304),
-    (RUN, 5, 9, 8, 1 << 20), (RUN, 3, 9, 32, 1 << 20),
-    # from 10 on: windows wider than 3.3 steps, 16384; steps 7 and 8 to range 11, 30000
+    (RUN, 4, 6, 8, 49151), (MFMA, 4, 6, 8, 49152), (RUN, 3, 9, 16, 49151), (MFMA, 3, 9, 16, 49152),
+    (RUN, 5, 5, 8, 1 << 20), (RUN, 5, 9, 8, 1 << 20), (RUN, 4, 5, 32, 1 << 20), (RUN, 3, 9, 32, 1 << 20),
+    # from 10 on: windows wider than 3.3 steps, 16384; steps 7 and 8 to range 11
+    # (12 at group 8), 30000
     (RUN, 6, 10, 32, 16383), (MFMA, 6, 10, 32, 16384), (RUN, 7, 10, 8, 29999), (MFMA, 7, 10, 8, 30000),
     (RUN, 8, 11, 32, 29999), (MFMA, 8, 11, 32, 30000), (RUN, 7, 11, 8, 29999), (MFMA, 7, 12, 8, 16384),
-    (RUN, 8, 12, 16, 1 << 20), (RUN, 8, 13, 16, 16383), (MFMA, 8, 13, 16, 16384), (RUN, 20, 10, 8, 1 << 20),
+    (RUN, 8, 12, 16, 1 << 20), (RUN, 8, 12, 8, 29999), (MFMA, 8, 12, 8, 30000), (RUN, 8, 13, 16, 16383),
+    (MFMA, 8, 13, 16, 16384), (RUN, 20, 10, 8, 1 << 20),
     # any range: small frames stay where the run matcher fits; groups of 64 never leave
     (RUN, 3, 18, 8, 6889), (RUN, 8, 18, 16, 1024), (MFMA, 3, 18, 8, 16384), (MFMA, 3, 40, 32, 100),
     (RUN, 3, 16, 64, 1 << 20), (WAVE, 3, 40, 64, 1 << 20)])

@@ -105,31 +105,32 @@ std::atomic<int> g_match_path{0};
 // each reference's own window, with its keys in registers up to range 17.
 // Times of the run matcher over the MFMA's at groups 8 / 16 (/ 32); content: a
 // noisy frame, one with a quarter of it constant bars, one half constant, and
-// a clean ramp in 8-bit steps. The first three lines keep all four at 1 or above:
-//   ranges up to 5, steps up to 4, from 49152 references on (57101, 1280 x 720
-//     at step 4, range 5): 1.28 / 1.08, 1.34 / 1.16, 1.35 / 1.24, 1.25 / 1.08;
-//     below (20437, 768 x 432) bars 1.10 / 0.99, ramp 1.22 / 1.03;
-//     smaller ranges and steps and larger frames gain more, to 3.2;
-//   ranges 6 to 9, from 98304 on (101575, 1280 x 720 at step 3, range 9): 1.49
-//     / 1.24, 1.32 / 1.17, 1.53 / 1.36, 1.39 / 1.19; 128851 (1080p, step 4)
-//     1.44 / 1.19, 1.38 / 1.20, 1.50 / 1.32, 1.36 / 1.12; below (57101, step 4)
-//     half constant 0.99 / 0.90; at group 32 noisy frames have 1.05 to 1.1;
+// a clean ramp in 8-bit steps. The first two lines keep all four at 1 or above:
+//   ranges up to 9, steps up to 4, from 49152 references on (57101, 1280 x 720
+//     at step 4, range 9): 1.33 / 1.04, 1.25 / 1.03, 1.26 / 1.05, 1.23 / 1.02;
+//     128851 (1080p, step 4) 1.43 / 1.17, 1.4 / 1.2, 1.5 / 1.3, 1.38 / 1.12;
+//     smaller ranges and steps and larger frames gain more, to 3.2; below
+//     (36465, 768 x 432 at step 3, range 9) half constant 0.94 / 0.76, but
+//     ranges up to 4 at group 8 have 1.1 to 1.3 from 16384 on (16899, 520 x 528
+//     at step 4, range 4: 1.11, 1.17, 1.18, 1.17); at group 32 noisy frames have
+//     1.05 to 1.1;
 //   steps 7 and 8 at ranges 10 and 11, from 30000 on (1080p, step 8, range 10):
 //     1.42 / 1.23 / 1.21, 1.40 / 1.24 / 1.14, 1.26 / 1.22 / 1.43, 1.35 / 1.24 /
 //     1.21; below (18755, 1280 x 720 at step 7, range 11) bars 1.05 / 0.93 /
-//     0.98; range 12 at step 8 1.12 / 0.96 / 1.01, bars 1.12 / 1.06 / 0.91;
+//     0.98; step 8, range 12 1.12 / 0.96 / 1.01, 1.12 / 1.06 / 0.91, 1.05 / 1.02
+//     / 1.15, 1.07 / 0.99 / 0.89: group 8 only;
 //   windows wider than 3.3 steps, from 16384 on: step 8, range 16 1.46 / 1.46 /
 //     1.40, step 3, range 16 2.7 / 2.4 / 2.2, step 3, range 19 4.4 / 3.8 / 2.5.
 //     Below, small launches leave the run matcher ahead on some content: 256 x
 //     256, step 3, range 18 2.2 / 1.8 / 0.67, with bars 0.6 / 0.5 / 0.7.
-// What none of the lines holds for is noise-free patchwork (squares of 24 or
-// 100 pixels, a value each): many exact copies overflow the lists, and from
-// range 7 on the run matcher is up to twice as fast.
+// What none of the lines holds for is noise-free patchwork, where many exact
+// copies overflow the lists: squares of 100 pixels, a value each, 1.0 / 0.9 at
+// step 3, range 7, squares of 24 0.78 / 0.64 there and half at range 9.
 bool match_mfma_pays(int step, int range, int group, long long nref) {
     if (group > 32) return false;
-    if (range < 10) return step <= 4 && group <= 16 && nref >= (range <= 5 ? 49152 : 98304);
+    if (range < 10) return step <= 4 && group <= 16 && nref >= (range <= 4 && group <= 8 ? 16384 : 49152);
     if (3 * (2 * range + 1) > 10 * step) return nref >= 16384;
-    return range <= 11 && step <= 8 && nref >= 30000;
+    return step <= 8 && (range <= 11 || (range == 12 && group <= 8)) && nref >= 30000;
 }
 
 int match_path() { return g_match_path.load(std::memory_order_relaxed); }
