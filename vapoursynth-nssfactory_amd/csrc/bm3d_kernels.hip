@@ -1504,11 +1504,14 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
     // by rounds of a wave minimum over each lane's four best. Windows that do
     // not fit come in pieces; the lanes carry the best so far. A window whose
     // first places hold G - 1 copies of the patch (distance 0) is done with
-    // those: no later place can displace one (flat areas). A wave looks through
-    // the first 64 of its own reference's, then all four through each other
-    // reference's next 256: against 256 by all at once, 1080p at step 3, range 7,
-    // group 8: half the frame constant 239 -> 181 us, squares of 100 pixels 450
-    // -> 310.
+    // those: no later place can displace one (flat areas). Windows of up to 400
+    // places (range 9): a wave looks through the first 64 of its own reference's,
+    // then all four through each other reference's next 256; against 256 by all
+    // at once, 1080p at step 3, range 7, group 8: half the frame constant 239 ->
+    // 181 us, squares of 100 pixels 450 -> 310. Wider ones go to the 256 at
+    // once: theirs are mostly denoised planes, whose lists overflow without
+    // copies, and the first look cost them 2 % (step 8, range 19, group 32:
+    // 376 -> 386 us of both stages' matching).
     const int space = reg_words + kUnion;
     const int wcap = min((2 * jb.range + 1) * (2 * jb.range + 1), (ux1 - ux0 + 1) * (uy1 - uy0 + 1));
     const int at_once = max(1, min(4, space / wcap));
@@ -1559,8 +1562,8 @@ __global__ __launch_bounds__(256, 5) void match_mfma_kernel(MatchTable tab) {
             if (p0 == 0) {
                 // (a reference done after 64 places has its copies among them:
                 // its keys from there to `from` are not written and not read)
-                for (int pass = 0; pass < 2 && flat != (1u << nref) - 1u; ++pass) {
-                    const int next = min(piece, pass == 0 ? 64 : 320);
+                for (int pass = wcap <= 400 ? 0 : 1; pass < 2 && flat != (1u << nref) - 1u; ++pass) {
+                    const int next = min(piece, pass == 0 ? 64 : from + 256);
                     for (int r = 0; r < nref; ++r)
                         if (pass == 0 ? r == wave : !((flat >> r) & 1u)) {
                             const int zeros = score(r, 0, from, next, pass == 0);
