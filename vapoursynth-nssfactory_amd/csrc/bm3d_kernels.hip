@@ -799,16 +799,20 @@ __global__ __launch_bounds__(64) void match_wave_kernel(MatchTable tab) {
 // carry (non-finite, or |v - mu| >= 8192 so that S would be negative), scores
 // its whole window exactly. A region of one value needs no scores at all.
 //
-// What bounds it: VALU issue and the matrix unit together (per wave of the
-// step-3, range-16, group-16 launch 3.05 k VALU instructions against 6.0 k with
-// the norms, masks and rank sums on the VALU, and 186 MFMAs; about 80 % of the
-// SIMDs' cycles; the passes take 60 % of the time). Per
-// 1080p YUV420 frame at step 3, range 16: group 16 on the noisy planes 660 us
-// (1115 before the norms and masks went into the MFMAs, the sums of ranks into
-// row minima and the reference's patch into registers), group 32 on the
-// denoised ones 1060 us (1758); gray 1080p, step 8, range 30, group 16: 258 us
-// (468). Lists of 160 cost 1340 us at group 32 (overflows), of 256 1126 (LDS:
-// four workgroups per CU instead of five).
+// What bounds it: VALU issue and the matrix unit together. Per wave of the 1080p
+// YUV420, step-3, range-19, group-16 launch 3.25 k VALU instructions, 211 MFMAs
+// among them (with the norms, masks and rank sums on the VALU 6.0 k at range 16
+// already): 0.8 of the two a CU can issue per cycle, the matrix units busy 27 %
+// of the time, 28 % of the wave cycles waiting. At range 30 (7.2 k, 737) 0.6,
+// 34 % and 30 %: 56 KB of LDS leave two workgroups per CU. The bound of five
+// workgroups per CU spills four registers (20 bytes of scratch per lane).
+// Per 1080p YUV420 frame at step 3, range 16: group 16 on the noisy planes 627
+// us (1115 before the norms and masks went into the MFMAs, the sums of ranks into
+// row minima and the reference's patch into registers); gray 1080p, step 8, range
+// 30, group 16: 244 us (468). Group 32 on denoised planes took 1060 us (1758);
+// lists of 160 cost 1340 there (overflows), of 256 1126 (LDS: four workgroups per
+// CU instead of five). A constant 1080p plane at step 3, range 16: 59 us (the run
+// matcher 828).
 //
 // Error bound, in the scaled units (every distance times 2^2S; u = 2^-24):
 //   per element, |(v - mu) 2^S - h| <= 2^-11 |h| (1 + 2^-11) for a normal h,
@@ -3315,10 +3319,11 @@ __global__ __launch_bounds__(256) void filter_temporal_b8_kernel(TFilterTable ta
     }
 }
 
-// Temporal tile path, block 8, G in {8, 16, 32}: 8 waves per workgroup, a
-// wave per group with the register cube; every slot's contributions go into
-// that slot's LDS sums (apron = the slot's reach around the tile), then out as
-// the centre's float partials, slot by slot. The LDS (well over half a CU's)
+// Temporal tile path, block 8, G in {8, 16, 32}: 8 waves per workgroup (16 at
+// groups of 8 where the slots leave one workgroup per CU), a wave per group with
+// the register cube; every slot's contributions go into that slot's LDS sums
+// (apron = the slot's reach around the tile), then out as the centre's float
+// partials, slot by slot. The LDS (well over half a CU's)
 // leaves one workgroup per CU, so the kernel is persistent: workgroup L (in
 // XCD-contiguous order) filters tiles [L T / n, (L + 1) T / n) of the T tiles,
 // and while one tile's partials are written it loads the next tile's records
@@ -4361,9 +4366,12 @@ __global__ __launch_bounds__(64) void ncsr_group_kernel(WnnmTable tab) {
 //            groups (77 G/s: 218 us for the 16.6 M of 32 400 groups of 8).
 // Measured on a 1080p plane (MI355X; gram_group_body with its atomics before):
 // groups of 8, step 8 (32 400): 215 -> 59 us, NCSR 225 -> 67 us; groups of 16,
-// step 4 (128 855): 3 732 -> 984 us, there bound by VALU issue in the rounds
-// (96 % of the SIMDs' cycles); the smaller launch holds four waves per SIMD and
-// waits a third of its cycles.
+// step 4 (128 855): 3 732 -> 984 us. There VALU issue in the rounds bounds it: 17
+// k instructions per wave, 1.04 of the two a CU can issue per cycle, 19 % of the
+// wave cycles waiting. The smaller launch holds four waves per SIMD and waits a
+// third of its cycles. The selects' masks
+// take all scalar registers at groups of 16: 25 (NCSR 26) of them spill, and the
+// WNNM kernel keeps 36 bytes of scratch per lane.
 // ---------------------------------------------------------------------------
 
 // rr_partner for a full group.
